@@ -418,8 +418,9 @@ extern "C" int motif_gdn_recurrent_fwd(
 
 extern "C" size_t motif_gdn_chunk_workspace_bytes(int H, int dk, int dv, int chunk, int total_chunks) {
   if (H <= 0 || dk <= 0 || dv <= 0 || chunk <= 0 || total_chunks <= 0) return 0;
-  // bf16 inputs on the MFMA path need its layout; fp32 inputs use the fp32 kernels.
+  // whichever of the bf16 MFMA, fp32 MFMA and vector kernels serves the inputs
   size_t mfma = chunk_mfma_supported(dk, dv, chunk) ? chunk_mfma_workspace_bytes(H, dk, dv, total_chunks) : 0;
+  // (the fp32 MFMA kernels' dk dk + dk dv + 64 dk floats are within the vector kernels' share)
   const size_t per = static_cast<size_t>(chunk) * (1 + dk + dv + chunk);
   return std::max(mfma, per * H * total_chunks * sizeof(float));
 }
@@ -498,8 +499,11 @@ static int chunk_fwd_impl(
   if (in_dtype != MOTIF_F32 && in_dtype != MOTIF_BF16)
     return set_error(MOTIF_ERR_UNSUPPORTED, "gdn_chunk: unsupported dtype");
   // bf16 inputs take the MFMA path (3-pass bf16 products, ~16 mantissa bits);
-  // fp32 inputs keep fp32 FMA throughout (the 1e-4 accuracy mode).
+  // fp32 inputs keep fp32 multiplies and sums throughout (the 1e-4 accuracy mode).
   if (chunk_mfma_eligible(a, chunk, in_dtype, out_dtype)) return launch_chunk_mfma(a, ca, workspace, s);
+  if (in_dtype == MOTIF_F32 && chunk_f32_supported(dk, dv, chunk) && chunk_f32_workspace_bytes(H, dk, dv, total_chunks) <= need &&
+      (reinterpret_cast<uintptr_t>(workspace) & 15) == 0)
+    return launch_chunk_f32(a, ca, workspace, s);
   if (in_dtype == MOTIF_F32) return launch_chunk<float>(a, ca, chunk, s);
   if (in_dtype == MOTIF_BF16) return launch_chunk<bf16_t>(a, ca, chunk, s);
   return set_error(MOTIF_ERR_UNSUPPORTED, "gdn_chunk: unsupported dtype");

@@ -15,6 +15,7 @@
 // this path in fp32 (tf32x3 products).
 #include "capi_internal.h"
 #include "common.h"
+#include "gdn_internal.h"
 
 namespace motif {
 
@@ -277,6 +278,11 @@ struct OpScanArgs {
   const float *M, *Q, *s0;  // [BH][N][DK][DK], [BH][N][DK][Dv], [BH][DK][Dv] or null
   float *rec, *s_out;       // [BH][N][DK][Dv], [BH][DK][Dv]
   int N, Dv, BH, rev;
+  // CELLS form (launch_opscan_cells), cells by [head][chunk]: state bh = sequence * H + head
+  // starts at cell head * total + sequence * N, or with coff at head * total + coff[sequence]
+  // with coff[sequence + 1] - coff[sequence] chunks.  Other forms: cells by [bh][chunk].
+  int H, total;
+  const int32_t *coff;
 };
 template <int DK> constexpr int opscan_ms() { return DK + 4; }  // LDS row stride (floats) of M and S^T
 // workgroups of one scan: whole groups of column-group workgroups per XCD
@@ -284,14 +290,17 @@ inline int opscan_blocks(int BH, int Dv) { return (BH + kXcds - 1) / kXcds * kXc
 
 // One scan on workgroup `id` of its launch range, with the caller's LDS: sM [2][DK * MS]
 // and sS [2][16 * MS] floats.
-template <int DK, bool TRANS>
+template <int DK, bool TRANS, bool CELLS = false>
 __device__ __forceinline__ void opscan_body(const OpScanArgs &oa, int id, float (*sM)[DK * opscan_ms<DK>()],
                                             float (*sS)[kCols * opscan_ms<DK>()]) {
   constexpr int TT = DK / 16, MS = opscan_ms<DK>();  // row tiles; LDS row stride
   using PR = OpPre<DK>;
-  const float *__restrict__ M = oa.M, *__restrict__ Q = oa.Q, *__restrict__ s0 = oa.s0;
-  float *__restrict__ rec = oa.rec, *__restrict__ s_out = oa.s_out;
-  const int N = oa.N, Dv = oa.Dv, BH = oa.BH, rev = oa.rev;
+  // (CELLS: rec may be Q -- each lane reads an element of Q_n kOpDepth chunks before it
+  // overwrites that element with S_n -- so neither is restrict)
+  const float *__restrict__ M = oa.M, *Q = oa.Q, *__restrict__ s0 = oa.s0;
+  float *rec = oa.rec, *__restrict__ s_out = oa.s_out;
+  int N = oa.N;
+  const int Dv = oa.Dv, BH = oa.BH, rev = oa.rev;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int lr = lane & 15, lq = lane >> 4;
   // linear id L on XCD L % 8: slot L / 8 of that XCD holds column group slot % ncg of
@@ -300,9 +309,15 @@ __device__ __forceinline__ void opscan_body(const OpScanArgs &oa, int id, float 
   const int bh = (slot / ncg) * kXcds + id % kXcds, v0 = (slot % ncg) * kCols;
   if (bh >= BH) return;
   const size_t mstride = static_cast<size_t>(DK) * DK, qstride = static_cast<size_t>(DK) * Dv;
-  const float *Mb = M + static_cast<size_t>(bh) * N * mstride;
-  const float *Qb = Q + static_cast<size_t>(bh) * N * qstride;
-  float *recb = rec + static_cast<size_t>(bh) * N * qstride;
+  size_t cell = static_cast<size_t>(bh) * N;
+  if constexpr (CELLS) {
+    const int sq = bh / oa.H, hd = bh % oa.H;
+    cell = static_cast<size_t>(hd) * oa.total + (oa.coff ? oa.coff[sq] : sq * N);
+    if (oa.coff) N = oa.coff[sq + 1] - oa.coff[sq];
+  }
+  const float *Mb = M + cell * mstride;
+  const float *Qb = Q + cell * qstride;
+  float *recb = rec + cell * qstride;
   auto order = [&](int i) { return rev ? N - 1 - i : i; };
 
   // element (row, col) of a state-shaped [DK][Dv] matrix held by this lane for tile m, r
@@ -402,11 +417,11 @@ __device__ __forceinline__ void opscan_body(const OpScanArgs &oa, int id, float 
   }
 }
 
-template <int DK, bool TRANS>
+template <int DK, bool TRANS, bool CELLS>
 __global__ void __launch_bounds__(256) gdn_opscan_f32_kernel(OpScanArgs oa) {
   __shared__ __attribute__((aligned(16))) float sM[2][DK * opscan_ms<DK>()];
   __shared__ __attribute__((aligned(16))) float sS[2][kCols * opscan_ms<DK>()];
-  opscan_body<DK, TRANS>(oa, blockIdx.x, sM, sS);
+  opscan_body<DK, TRANS, CELLS>(oa, blockIdx.x, sM, sS);
 }
 
 // Both scans of the backward in one launch (they are independent: the reverse scan needs
@@ -430,6 +445,17 @@ int check_scan_sizes(int BH, int N, int C, int Dk, int Dv, const char *who) {
 }
 
 }  // namespace
+
+int launch_opscan_cells(const float *A, float *Hn, const float *s_in, float *s_out, int H, const ChunkArgs &ca, int dk,
+                        int dv, hipStream_t s) {
+  const int BH = ca.nseq * H;
+  const OpScanArgs oa{A, Hn, s_in, Hn, s_out, ca.nper, dv, BH, 0, H, ca.total_chunks, ca.coff};
+  const dim3 grid(opscan_blocks(BH, dv)), block(256);
+  if (dk == 64) gdn_opscan_f32_kernel<64, false, true><<<grid, block, 0, s>>>(oa);
+  else if (dk == 32) gdn_opscan_f32_kernel<32, false, true><<<grid, block, 0, s>>>(oa);
+  else return set_error(MOTIF_ERR_UNSUPPORTED, "gdn_opscan: dk must be 32 or 64");
+  return check_launch("gdn_opscan_f32_kernel");
+}
 
 }  // namespace motif
 
@@ -472,8 +498,8 @@ extern "C" int motif_gdn_opscan_f32(const float *M, const float *Q, const float 
   if (reinterpret_cast<uintptr_t>(M) & 15) return set_error(MOTIF_ERR_UNSUPPORTED, "gdn_opscan_f32: M needs 16-byte alignment");
   const dim3 grid(opscan_blocks(BH, Dv)), block(256);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const OpScanArgs oa{M, Q, S0, rec, S_out, N, Dv, BH, reverse};
-#define MOTIF_OPSCAN(D, T) gdn_opscan_f32_kernel<D, T><<<grid, block, 0, s>>>(oa)
+  const OpScanArgs oa{M, Q, S0, rec, S_out, N, Dv, BH, reverse, 0, 0, nullptr};
+#define MOTIF_OPSCAN(D, T) gdn_opscan_f32_kernel<D, T, false><<<grid, block, 0, s>>>(oa)
   if (Dk == 16) { if (transpose) MOTIF_OPSCAN(16, true); else MOTIF_OPSCAN(16, false); }
   else if (Dk == 32) { if (transpose) MOTIF_OPSCAN(32, true); else MOTIF_OPSCAN(32, false); }
   else { if (transpose) MOTIF_OPSCAN(64, true); else MOTIF_OPSCAN(64, false); }
@@ -496,7 +522,8 @@ extern "C" int motif_gdn_opscan_pair_f32(const float *A, const float *Hn, const 
   const int g1 = opscan_blocks(BH, Dv);
   const dim3 grid(2 * g1), block(256);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const OpScanArgs fwd{A, Hn, S0, P, S_out, N, Dv, BH, 0}, rev{A, G, dS_final, dSn, dS0, N, Dv, BH, 1};
+  const OpScanArgs fwd{A, Hn, S0, P, S_out, N, Dv, BH, 0, 0, 0, nullptr},
+      rev{A, G, dS_final, dSn, dS0, N, Dv, BH, 1, 0, 0, nullptr};
   if (Dk == 16) gdn_opscan_pair_f32_kernel<16><<<grid, block, 0, s>>>(fwd, rev, g1);
   else if (Dk == 32) gdn_opscan_pair_f32_kernel<32><<<grid, block, 0, s>>>(fwd, rev, g1);
   else gdn_opscan_pair_f32_kernel<64><<<grid, block, 0, s>>>(fwd, rev, g1);

@@ -72,4 +72,16 @@ size_t chunk_mfma_workspace_bytes(int H, int dk, int dv, int total_chunks);
 bool chunk_mfma_eligible(const GdnArgs &a, int chunk, int in_dtype, int out_dtype);
 int launch_chunk_mfma(const GdnArgs &a, const ChunkArgs &ca, void *workspace, hipStream_t s);
 
+// fp32 MFMA chunk path (gdn_f32.hip): fp32 in and out, any row alignment; 16-byte aligned
+// workspace.
+bool chunk_f32_supported(int dk, int dv, int chunk);
+size_t chunk_f32_workspace_bytes(int H, int dk, int dv, int total_chunks);
+int launch_chunk_f32(const GdnArgs &a, const ChunkArgs &ca, void *workspace, hipStream_t s);
+
+// S <- A_n S + H_n over the chunks of every (sequence, head) (gdn_bwd.hip): A [cells][dk][dk],
+// Hn [cells][dk][dv] by cell head * total_chunks + chunk, s_in / s_out [nseq][H][dk][dv]
+// (s_in NULL: zeros).  Every S_n goes over H_n.
+int launch_opscan_cells(const float *A, float *Hn, const float *s_in, float *s_out, int H, const ChunkArgs &ca, int dk,
+                        int dv, hipStream_t s);
+
 }  // namespace motif
