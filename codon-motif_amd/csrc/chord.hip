@@ -13,6 +13,8 @@
 // GGD bias depends only on d = key - i_abs: each wave evaluates it in registers (one new
 // distance per lane per tile) into an LDS window; no bias is stored in HBM.
 //
+// chord_wide_kernel (chord_wide.hip): the prefill of every other type and head dim.
+//
 // chord_decode_kernel (decode / short queries over a long cache): split-K
 // flash-decoding.  A workgroup owns (split, kv head, batch row) and serves all
 // query rows of that kv head (GQA group x L <= 8), streaming K and V with fully
@@ -27,28 +29,6 @@
 #include "common.h"
 
 namespace motif {
-
-struct ChordArgs {
-  const void *q; int64_t q_sb, q_sh, q_st;
-  const void *k; int64_t k_sb, k_sh, k_st;
-  const void *v; int64_t v_sb, v_sh, v_st;
-  const float *alpha, *beta, *mu, *ssmax;
-  const float *log_n; int64_t ln_sb, ln_st;
-  void *out; int64_t o_sb, o_sh, o_st;
-  float *lse;
-  int B, H, Hkv, L, S, q_start;
-  float scale, eps;
-  const int32_t *cu;  // packed sequences (B == 1) or nullptr
-  // split-K partials
-  float *part;        // [B][Hkv][splits][L * group][D + 2]
-  int splits;         // key-range splits (decode kernel)
-  int nqc;            // row chunks per (batch, kv head) (decode kernel)
-  // device cursor (decode kernels): when set, *len_dev positions are cached, the L
-  // new keys sit at [*len_dev, *len_dev + L), S holds the cache capacity, and the
-  // merge pass advances *len_dev by L
-  int *len_dev;
-  const float *log_tab;  // ln(1 .. n) when log_n is NULL: log_n[b, i] = log_tab[q_start + i]
-};
 
 // Keys and query start of a decode launch: from the host arguments, or from the
 // device cursor (clamped so the window stays inside the capacity).
@@ -65,12 +45,6 @@ __device__ __forceinline__ float log_n_at(const ChordArgs &a, int b, int i, int 
 
 constexpr int kD = 64;        // head dim
 constexpr int kBN = 64;       // keys per tile
-
-__device__ __forceinline__ float ggd_bias(float dist, float alpha, float beta, float mu, float eps) {
-  // -alpha * (|d - mu| + eps)^beta, the power through exp2(beta * log2(.)).
-  const float x = fabsf(dist - mu) + eps;
-  return -alpha * fast_exp2(beta * fast_log2(x));
-}
 
 __device__ __forceinline__ __bf16 to_bf(float f) {
   const bf16_t b = f32_to_bf16(f);
@@ -574,8 +548,9 @@ constexpr int kDecKeys = 4;                 // keys per lane group per step
 // K / V rows and bias entries are loaded before the current step is computed (two
 // register stages), so a wave keeps a step of loads in flight.  Each lane group keeps
 // its own running max / sum / output (merged at the end): the step has no cross-lane
-// traffic besides the LPK-lane dot-product sums.  This kernel serves every dtype
-// (fp32, bf16, fp16) and head dim (16, 32, 64, 128); bf16 at D = 64 has MFMA kernels.
+// traffic besides the LPK-lane dot-product sums.  This kernel serves the decode steps of
+// every dtype (fp32, bf16, fp16) and head dim (16, 32, 64, 128) -- bf16 at D = 64 has an MFMA
+// kernel -- and the prefills whose row strides chord_wide.hip does not take.
 template <typename T, int R, int D>
 __global__ void __launch_bounds__(256) chord_decode_kernel(ChordArgs a, const float *tab, int tab_n) {
   constexpr int LPK = D / 8, KG = 64 / LPK, kDecStep = KG * kDecKeys;
@@ -1334,6 +1309,11 @@ extern "C" int motif_chord_fwd(
     const size_t need = tb + (a.splits > 1 ? static_cast<size_t>(B) * Hkv * a.splits * rows * (D + 2) * sizeof(float) : 0);
     if (!workspace || workspace_bytes < need)
       return set_error(MOTIF_ERR_INVALID, "chord_fwd: workspace too small (need " + std::to_string(need) + " bytes)");
+    // more rows than a decode step: the fp32-arithmetic flash kernel, unless its 32-bit tile
+    // offsets are too small for the row strides.  The vector kernel has no key split there and
+    // loses from its smallest call on: 12 heads, 3 kv heads, fp32, 3 tokens over 300: 27 against
+    // 30 us through the op; 3 over 4096: 85 against 102; 9 over 33 with 12 kv heads: 27 against 29.
+    if (!use_decode(H, Hkv, L, packed) && chord_wide_serves(a)) return launch_chord_wide(a, dtype, D, s);
     float *tab = static_cast<float *>(workspace);
     if (a.splits > 1) a.part = reinterpret_cast<float *>(static_cast<char *>(workspace) + tb);
     const int tn = table_len(S);

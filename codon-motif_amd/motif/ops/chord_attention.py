@@ -3,10 +3,11 @@
 `apply_chord_attention` keeps the reference signature, defaults, validation
 messages and exception types (motif/ops/chord_attention.py:1557-1625 with
 `_check_tensors` :966-1011 and `_check_params` :1448-1472).  The launcher
-picks the bf16 MFMA flash kernel for prefill shapes and the split-K vector
-kernel when a kv head serves at most 8 query rows (GQA group x L), which is
-the reference's long-KV / short-Q split path (:1128-1229).  fp32 inputs run on
-the vector kernel for every shape (fp32 FMA throughout, the accuracy mode).
+picks the bf16 MFMA flash kernel for prefill shapes (head dim 64; other head dims,
+fp16 and fp32 the fp32-arithmetic flash kernel) and the split-K decode kernels when
+a kv head serves at most 8 query rows (GQA group x L), which is the reference's
+long-KV / short-Q split path (:1128-1229).  fp32 inputs are multiplied and summed in
+fp32 on every path (the accuracy mode).
 `apply_chord_attention_varlen` adds packed sequences (new) and
 `chord_decode_cursor` the decode step over a fixed-capacity cache whose length
 lives on the device (new; the graph-replayable form of the decode call).
@@ -25,7 +26,7 @@ from .packed import PackedSeqs
 from .autograd_path import chord_attention_torch, chord_attention_varlen_torch, wants_grad
 
 HEAD_DIM = 64                  # the model's head dim: bf16 runs on the MFMA kernels
-HEAD_DIMS = (16, 32, 64, 128)  # head dims the kernels serve (fp32 / fp16 / other D: the vector kernel)
+HEAD_DIMS = (16, 32, 64, 128)  # head dims the kernels serve
 
 
 def serves_head_dim(D: int) -> bool:
