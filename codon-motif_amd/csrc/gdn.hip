@@ -501,9 +501,7 @@ static int chunk_fwd_impl(
   // bf16 inputs take the MFMA path (3-pass bf16 products, ~16 mantissa bits);
   // fp32 inputs keep fp32 multiplies and sums throughout (the 1e-4 accuracy mode).
   if (chunk_mfma_eligible(a, chunk, in_dtype, out_dtype)) return launch_chunk_mfma(a, ca, workspace, s);
-  if (in_dtype == MOTIF_F32 && chunk_f32_supported(dk, dv, chunk) && chunk_f32_workspace_bytes(H, dk, dv, total_chunks) <= need &&
-      (reinterpret_cast<uintptr_t>(workspace) & 15) == 0)
-    return launch_chunk_f32(a, ca, workspace, s);
+  if (in_dtype == MOTIF_F32 && chunk_f32_eligible(a, chunk, workspace)) return launch_chunk_f32(a, ca, workspace, s);
   if (in_dtype == MOTIF_F32) return launch_chunk<float>(a, ca, chunk, s);
   if (in_dtype == MOTIF_BF16) return launch_chunk<bf16_t>(a, ca, chunk, s);
   return set_error(MOTIF_ERR_UNSUPPORTED, "gdn_chunk: unsupported dtype");

@@ -17,6 +17,7 @@
 // at H = 12, T = 4096, dv = 128 (78 + 54 + 20; was 1220).  The prep is bound by its MFMA chains
 // and the LDS round trips between its phases (one workgroup per CU), the scan by the chain.
 // Its error against 64 bits is the smaller one too (2.4e-7 against 2.8e-7 relative).
+#include <algorithm>
 #include <type_traits>
 
 #include "gdn_internal.h"
@@ -44,44 +45,6 @@ struct F32Lds {
   static constexpr int gam = at + kC * kLT, eg = gam + kC, kd = eg + kC, be = kd + kC, xs = be + kC;
   static constexpr int floats = xs + 32 * 33;
 };
-
-// A chunk's rows (cols of them valid, the rest of COLS zero) in registers, zero past len:
-// every load of the workgroup's matrices is issued before the first LDS store.
-template <int COLS>
-struct F32Rows {
-  static constexpr int q4 = COLS / 4, n = kC * q4 / kThreads;
-  static_assert(kC * q4 % kThreads == 0, "whole float4 rounds per thread");
-  f32x4 x[n];
-};
-template <int COLS>
-__device__ __forceinline__ F32Rows<COLS> f32_fetch(const float *src, int64_t st, int len, int cols, bool vec) {
-  using R = F32Rows<COLS>;
-  R rw;
-#pragma unroll
-  for (int j = 0; j < R::n; ++j) {
-    const int e = threadIdx.x + kThreads * j, r = e / R::q4, c = 4 * (e - r * R::q4);
-    const float *p = src + int64_t(min(r, len - 1)) * st + min(c, cols - 4);
-    if (vec) {
-      rw.x[j] = *reinterpret_cast<const f32x4 *>(p);
-    } else {
-#pragma unroll
-      for (int t = 0; t < 4; ++t) rw.x[j][t] = p[t];
-    }
-  }
-  return rw;
-}
-template <int COLS, typename F>
-__device__ __forceinline__ void f32_put(float *dst, int ld, const F32Rows<COLS> &rw, int len, int cols, F scale) {
-  using R = F32Rows<COLS>;
-#pragma unroll
-  for (int j = 0; j < R::n; ++j) {
-    const int e = threadIdx.x + kThreads * j, r = e / R::q4, c = 4 * (e - r * R::q4);
-    const bool ok = r < len && c < cols;
-    const float s = scale(r);
-#pragma unroll
-    for (int t = 0; t < 4; ++t) dst[r * ld + c + t] = ok ? rw.x[j][t] * s : 0.f;
-  }
-}
 
 // sum over k in [0, K) of fa(k) fb(k) for a 32x32 tile, fa / fb the lane's row and column
 // (offset by the lane half): the two halves of the range in two independent chains, which
@@ -117,8 +80,17 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
     const int64_t row = min(lane, ci.len - 1);
     const float gr = static_cast<const float *>(a.g)[ci.batch * a.g_sb + hd * a.g_sh + (ci.t0 + row) * a.g_st];
     const float br = static_cast<const float *>(a.beta)[ci.batch * a.b_sb + hd * a.b_sh + (ci.t0 + row) * a.b_st];
-    const F32Rows<DK> rk = f32_fetch<DK>(kb, a.k_st, ci.len, DK, vec), rq = f32_fetch<DK>(qb, a.q_st, ci.len, DK, vec);
-    const F32Rows<DV> rv = f32_fetch<DV>(vb, a.v_st, ci.len, a.dv, vec);
+    TileRows<float, DK, kThreads> rk, rq;
+    TileRows<float, DV, kThreads> rv;
+    if (vec) {
+      rk.fetch(kb, a.k_st, ci.len, DK);
+      rq.fetch(qb, a.q_st, ci.len, DK);
+      rv.fetch(vb, a.v_st, ci.len, a.dv);
+    } else {
+      rk.template fetch<false>(kb, a.k_st, ci.len, DK);
+      rq.template fetch<false>(qb, a.q_st, ci.len, DK);
+      rv.template fetch<false>(vb, a.v_st, ci.len, a.dv);
+    }
     float s = lane < ci.len ? gr : 0.f;
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
@@ -132,10 +104,10 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
       sKd[lane] = exp_f(__shfl(s, 63, 64) - s);
       sB[lane] = be;
     }
-    f32_put<DK>(sK, LK, rk, ci.len, DK, [](int) { return 1.f; });
-    f32_put<DK>(sQ, LK, rq, ci.len, DK, [](int) { return 1.f; });
+    rk.put(sK, LK, ci.len, DK);
+    rq.put(sQ, LK, ci.len, DK);
     __syncthreads();
-    f32_put<DV>(sV, LV, rv, ci.len, a.dv, [&](int r) { return sB[r]; });  // V' = beta V
+    rv.put(sV, LV, ci.len, a.dv, [&](int r) { return sB[r]; });  // V' = beta V
   }
 
   // N = -strict(beta K K^T * D) (waves 0-2) and Attn = (Q K^T) * D (waves 4-6), the lower
@@ -307,6 +279,11 @@ int launch_f32_prep(const GdnArgs &a, const ChunkArgs &ca, const F32Ws &ws, int 
 // vector kernels of gdn.hip keep the other shapes.
 bool chunk_f32_supported(int dk, int dv, int chunk) {
   return chunk == kC && (dk == 32 || dk == 64) && dv % 32 == 0 && dv > 0 && dv <= 128;
+}
+bool chunk_f32_eligible(const GdnArgs &a, int chunk, const void *workspace) {
+  const int64_t lo = std::min({a.q_st, a.k_st, a.v_st}), hi = std::max({a.q_st, a.k_st, a.v_st});
+  return chunk_f32_supported(a.dk, a.dv, chunk) && lo >= 0 && hi < kTileMaxStride &&
+         (reinterpret_cast<uintptr_t>(workspace) & 15) == 0;
 }
 
 size_t chunk_f32_workspace_bytes(int H, int dk, int dv, int total_chunks) {

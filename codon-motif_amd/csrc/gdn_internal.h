@@ -72,9 +72,10 @@ size_t chunk_mfma_workspace_bytes(int H, int dk, int dv, int total_chunks);
 bool chunk_mfma_eligible(const GdnArgs &a, int chunk, int in_dtype, int out_dtype);
 int launch_chunk_mfma(const GdnArgs &a, const ChunkArgs &ca, void *workspace, hipStream_t s);
 
-// fp32 MFMA chunk path (gdn_f32.hip): fp32 in and out, any row alignment; 16-byte aligned
-// workspace.
+// fp32 MFMA chunk path (gdn_f32.hip): fp32 in and out, any row alignment, row strides within the
+// 32-bit offsets of its loads, a 16-byte aligned workspace.
 bool chunk_f32_supported(int dk, int dv, int chunk);
+bool chunk_f32_eligible(const GdnArgs &a, int chunk, const void *workspace);
 size_t chunk_f32_workspace_bytes(int H, int dk, int dv, int total_chunks);
 int launch_chunk_f32(const GdnArgs &a, const ChunkArgs &ca, void *workspace, hipStream_t s);
 

@@ -45,6 +45,127 @@ __device__ __forceinline__ void mm_pipe(f32x16 (&acc)[NP], OP op) {
   }
 }
 
+// The same with a rolled loop, for kernels whose accumulators leave no room for a fully unrolled
+// body's addresses: STEPS k-steps in blocks of U, two blocks per iteration.
+template <int STEPS, int NP, typename OP>
+__device__ __forceinline__ void mm_loop(f32x16 (&acc)[NP], OP op) {
+  constexpr int U = NP == 1 ? 4 : 2;
+  static_assert(STEPS % (2 * U) == 0, "whole block pairs");
+  float a[2][U][NP], b[2][U][NP];
+  auto read = [&](int buf, int s0) {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int p = 0; p < NP; ++p) op(p, s0 + u, a[buf][u][p], b[buf][u][p]);
+  };
+  auto mul = [&](int buf) {
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int p = 0; p < NP; ++p) acc[p] = mfma32_f32(a[buf][u][p], b[buf][u][p], acc[p]);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  read(0, 0);
+#pragma unroll 1
+  for (int s = 0; s < STEPS; s += 2 * U) {
+    read(1, s + U);
+    mul(0);
+    read(0, s + 2 * U < STEPS ? s + 2 * U : 0);  // (the last iteration's repeat is not used)
+    mul(1);
+  }
+}
+
+// A chunk's 64 rows of COLS elements of type T (the first `cols` of them valid) in registers, four
+// per piece, by NT threads: every load of a workgroup's matrices is issued before the first LDS
+// store.  Rows past len repeat the last valid one and are zeroed by put.  VEC: rows start on
+// four-element boundaries.  Offsets from the (uniform) first row are 32-bit: st below kTileMaxStride.
+constexpr int64_t kTileMaxStride = int64_t(1) << 23;
+template <typename T, int COLS, int NT>
+struct TileRows {
+  static constexpr int q4 = COLS / 4, n = 64 * q4 / NT;
+  static_assert(64 * q4 % NT == 0, "whole pieces per thread");
+  typedef T vec4 __attribute__((ext_vector_type(4)));
+  vec4 x[n];
+  template <bool VEC = true>
+  __device__ __forceinline__ void fetch(const T *src, int64_t st, int len, int cols) {
+    const char *base = reinterpret_cast<const char *>(src);
+#pragma unroll
+    for (int j = 0; j < n; ++j) {
+      const int e = threadIdx.x + NT * j, r = e / q4, c = 4 * (e - r * q4);
+      const uint32_t off = (static_cast<uint32_t>(min(r, len - 1)) * static_cast<uint32_t>(st) + min(c, cols - 4)) * sizeof(T);
+      if (VEC) {
+        x[j] = *reinterpret_cast<const vec4 *>(base + off);
+      } else {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) x[j][t] = *reinterpret_cast<const T *>(base + off + t * sizeof(T));
+      }
+    }
+  }
+  template <typename F>
+  __device__ __forceinline__ void put(float *dst, int ld, int len, int cols, F scale) const {
+#pragma unroll
+    for (int j = 0; j < n; ++j) {
+      const int e = threadIdx.x + NT * j, r = e / q4, c = 4 * (e - r * q4);
+      const bool ok = r < len && c < cols;
+      const float s = scale(r);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const T v = x[j][t];
+        dst[r * ld + c + t] = ok ? ld_val(v) * s : 0.f;
+      }
+    }
+  }
+  __device__ __forceinline__ void put(float *dst, int ld, int len, int cols) const {
+    put(dst, ld, len, cols, [](int) { return 1.f; });
+  }
+  __device__ __forceinline__ static float ld_val(T v) { return motif::ld(&v); }
+};
+
+// 64 rows of COLS elements at row stride st >= COLS, as TileRows, through a range-checked buffer
+// over the first len rows: rows past them read zeros, so staging needs no clamps or selects (code
+// that a workgroup runs once is bound by its own fetch).
+template <typename T, int COLS, int NT>
+struct BufRows {
+  static constexpr int q4 = COLS / 4, n = 64 * q4 / NT;
+  static_assert(64 * q4 % NT == 0 && NT % q4 == 0, "whole pieces per thread, one column per thread");
+  uint4 x[n];
+  __device__ __forceinline__ void fetch(const T *src, int64_t st, int len) {
+    const buf_t buf = make_buf(src, static_cast<uint32_t>(((len - 1) * st + COLS) * sizeof(T)));
+    const uint32_t r = threadIdx.x / q4, c = 4 * (threadIdx.x % q4), step = static_cast<uint32_t>(NT / q4 * st * sizeof(T));
+    uint32_t off = (r * static_cast<uint32_t>(st) + c) * sizeof(T);
+#pragma unroll
+    for (int j = 0; j < n; ++j, off += step) {
+      if constexpr (sizeof(T) == 4) {
+        x[j] = buf_ld16(buf, off);
+      } else {
+        const uint2 u = buf_ld8(buf, off);
+        x[j] = uint4{u.x << 16, u.x & 0xffff0000u, u.y << 16, u.y & 0xffff0000u};
+      }
+    }
+  }
+  __device__ __forceinline__ void put(float *dst, int ld) const {
+    float *p = dst + threadIdx.x / q4 * ld + 4 * (threadIdx.x % q4);
+#pragma unroll
+    for (int j = 0; j < n; ++j) {
+      const uint32_t w[4] = {x[j].x, x[j].y, x[j].z, x[j].w};
+#pragma unroll
+      for (int t = 0; t < 4; ++t) p[j * (NT / q4) * ld + t] = __uint_as_float(w[t]);
+    }
+  }
+};
+
+// The entries of a 64-row vector at this lane's accumulator rows first + 8 (r / 4) + 4 h + r % 4.
+__device__ __forceinline__ void acc_rows(float (&x)[16], const float *v, int first) {
+  const int h = (threadIdx.x & 63) >> 5;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const f32x4 u = *reinterpret_cast<const f32x4 *>(v + first + 8 * q + 4 * h);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) x[4 * q + t] = u[t];
+  }
+}
+
 // T = (I - A)^{-1} of a strictly lower triangular 64 x 64 A, both in LDS with row stride
 // LD, by a workgroup of at least 256 threads (every thread calls it; it starts and ends
 // behind a barrier of its own).  16 x 16 diagonal blocks by substitution (one wave each),

@@ -6,13 +6,12 @@ The reference differentiates its chunk rule in three pieces
 (:180-260, the triangular solve differentiated in closed form), the scan
 `_FusedScanFunction.backward` (:727-765, a reverse scan kernel plus batched products) and
 the per-chunk output combination (autograd through :851-855).  `GDNChunkFunction` runs
-the same pieces: the two sequential scans are the HIP kernels `motif_gdn_scan_fwd_f32`
-(re-scan for the per-chunk states P and residuals X) and `motif_gdn_scan_bwd_f32` (the
-reverse scan), the per-chunk terms are the HIP kernels `motif_gdn_bwd_prep_f32` (the chunk factors, the
-inverse by blocked substitution and the output's upstream terms) and
-`motif_gdn_bwd_chunk_f32` (every gradient of the preparation, the scan products and the
-output combination) for chunk 64, dk 64 and dv 64 / 128; other shapes take the same
-formulas as batched fp32 torch products (`_backward_torch`).
+the same pieces: for chunk 64, dk 64 and dv 64 / 128 in one call (`motif_gdn_chunk_bwd`: the
+per-chunk operators, both scans in operator form, every gradient); other shapes take the HIP
+scans `motif_gdn_scan_fwd_f32` (re-scan for the per-chunk states P and residuals X) and
+`motif_gdn_scan_bwd_f32` (the reverse scan) around batched fp32 torch products
+(`_backward_torch`).  The pieces are also entry points of their own (`bwd_prep`, `opscan_pair`,
+`bwd_chunk`).
 
 Per chunk, with gamma the within-chunk cumulative log decay, D[i, j] = e^{gamma_i -
 gamma_j} (j <= i), Kb = beta k, Vb = beta v, A = -(Kb k^T * D) strictly lower,
@@ -229,19 +228,41 @@ def _back(t, like, L):
     return t.reshape(B, H, N * C, *t.shape[4:])[:, :, :L].to(like.dtype)
 
 
+def _rows4(t):
+    '''t [B, H, L, D] with unit feature stride and separate rows on four-element boundaries (the
+    backward kernels' range-checked row loads), strides within their 32-bit offsets.'''
+    ok = (_separate_rows(t) and all(s % 4 == 0 for s in t.stride()[:-1])
+          and t.data_ptr() % (4 * t.element_size()) == 0)
+    return t if ok else torch.empty(t.shape, dtype=t.dtype, device=t.device).copy_(t)
+
+
+def _separate_rows(t):
+    return t.stride(-1) == 1 and t.shape[-1] <= t.stride(2) < 1 << 23
+
+
 def _backward_kernels(q, k, v, beta, g, S0, do, dS_fin, C):
-    '''The backward on the HIP kernels: per-chunk terms, forward re-scan, reverse scan,
-    per-chunk gradients (four launches plus the input chunking).'''
-    L = q.shape[2]
-    pad = (C - L % C) % C
-    qc, kc, vc, doc = (_chunks(t, C, pad).contiguous() for t in (q, k, v, do))
-    bc, gc = (_chunks(t, C, pad).contiguous() for t in (beta, g))
-    W, U, gam, T, dX, A, Hn, G = bwd_prep(qc, kc, vc, bc, gc, doc, operators=True)
-    P, _, dSn, dS0 = opscan_pair(A, Hn, S0, G, dS_fin)
-    # (the residuals X_n = U_n - W_n P_n are formed inside the per-chunk kernel)
-    dq, dk, dv, dbeta, dg = bwd_chunk(qc, kc, vc, bc, gam, T, P, None, dSn, doc, dX, W=W, U=U)
-    return (_back(dq, q, L), _back(dk, k, L), _back(dv, v, L), _back(dbeta, beta, L), _back(dg, g, L),
-            None if S0 is None else dS0.to(S0.dtype))
+    '''The backward on the HIP kernels (motif_gdn_chunk_bwd: the chunk operators, both scans,
+    the gradients: three launches) from the caller's tensors to gradients laid out and
+    typed like them.'''
+    like = (q, k, v, beta, g)
+    B, H, L, Dk = q.shape
+    Dv = v.shape[-1]
+    dt = torch.bfloat16 if all(t.dtype == torch.bfloat16 for t in like) else torch.float32
+    ins = [t.to(dt) for t in (*like, do)]
+    ins = [_rows4(t) if t.dim() == 4 else t for t in ins]
+    grads = [torch.empty_like(t) for t in ins[:5]]
+    # (a gradient takes its input's layout; one the kernel's row stores cannot address, the default)
+    grads = [gr if gr.dim() == 3 or _separate_rows(gr) else torch.empty(gr.shape, dtype=dt, device=gr.device) for gr in grads]
+    S0f, dSf = (None if t is None else t.float().contiguous() for t in (S0, dS_fin))
+    dS0 = torch.empty(B, H, Dk, Dv, dtype=torch.float32, device=q.device)
+    lib = _lib.lib()
+    ws = torch.empty(max(int(lib.motif_gdn_chunk_bwd_workspace_bytes(B, H, L, Dk, Dv)), 1), dtype=torch.uint8,
+                     device=q.device)
+    rc = lib.motif_gdn_chunk_bwd(
+        *(x for t in ins for x in _lib.t4(t)), _lib.ptr(S0f), _lib.ptr(dSf), *(x for t in grads for x in _lib.t4(t)),
+        dS0.data_ptr(), B, H, L, Dk, Dv, _lib.dtype_code(dt), ws.data_ptr(), ws.numel(), _lib.stream_ptr(q.device))
+    _lib.check(rc, 'motif_gdn_chunk_bwd')
+    return (*(gr.to(t.dtype) for gr, t in zip(grads, like)), None if S0 is None else dS0.to(S0.dtype))
 
 
 def _backward_torch(q, k, v, beta, g, S0, do, dS_fin, C):

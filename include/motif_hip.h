@@ -138,6 +138,32 @@ int motif_gdn_opscan_pair_f32(const float *A, const float *Hn, const float *S0, 
                               const float *dS_final, float *dSn, float *dS0, int BH, int N, int Dk, int Dv,
                               void *stream);
 /*
+ * Gradients of motif_gdn_chunk_fwd (chunk 64) in one call: from its inputs q, k [B,H,L,dk],
+ * v [B,H,L,dv], beta, g [B,H,L], the output's gradient dout [B,H,L,dv] and the final state's
+ * dstate_out [B,H,dk,dv] (fp32, contiguous, or NULL: zeros), the gradients dq, dk, dv, dbeta,
+ * dg (the inputs' dtype) and dstate_in [B,H,dk,dv] (fp32, contiguous) of the initial state
+ * state_in (or NULL: zeros).  All arithmetic fp32.  Replaces the reference's
+ * _PrepareChunksFunction.backward, _FusedScanFunction.backward and the output combination's
+ * gradient (motif/ops/gated_deltanet.py:180-260, :727-765, :830-855).  dk == 64, dv in
+ * {64, 128}; dtype fp32 or bf16 for every tensor; unit feature strides, rows of q, k, v and
+ * dout on four-element boundaries; 16-byte aligned workspace.
+ */
+size_t motif_gdn_chunk_bwd_workspace_bytes(int B, int H, int L, int dk, int dv);
+int motif_gdn_chunk_bwd(const void *q, int64_t q_sb, int64_t q_sh, int64_t q_st,
+                        const void *k, int64_t k_sb, int64_t k_sh, int64_t k_st,
+                        const void *v, int64_t v_sb, int64_t v_sh, int64_t v_st,
+                        const void *beta, int64_t b_sb, int64_t b_sh, int64_t b_st,
+                        const void *g, int64_t g_sb, int64_t g_sh, int64_t g_st,
+                        const void *dout, int64_t o_sb, int64_t o_sh, int64_t o_st,
+                        const float *state_in, const float *dstate_out,
+                        void *dq, int64_t dq_sb, int64_t dq_sh, int64_t dq_st,
+                        void *dk_, int64_t dk_sb, int64_t dk_sh, int64_t dk_st,
+                        void *dv_, int64_t dv_sb, int64_t dv_sh, int64_t dv_st,
+                        void *dbeta, int64_t db_sb, int64_t db_sh, int64_t db_st,
+                        void *dg, int64_t dg_sb, int64_t dg_sh, int64_t dg_st, float *dstate_in,
+                        int B, int H, int L, int dk, int dv, int dtype, void *workspace, size_t workspace_bytes,
+                        void *stream);
+/*
  * Chunk backward, the per-chunk terms before the scans (fp32).  Inputs are chunked and
  * zero-padded: q, k [BH,N,C,Dk], v, dout [BH,N,C,Dv], beta, g [BH,N,C].  Writes
  * gam = cumsum(g) per chunk [BH,N,C], T = (I + strict(beta k k^T * D))^{-1} [BH,N,C,C],
