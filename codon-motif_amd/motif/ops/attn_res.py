@@ -65,8 +65,7 @@ def attn_res_read(sources, query, norm):
     weight = norm.weight
     if weight is None:
         weight = torch.ones(D, dtype=dt, device=x0.device)
-    q = query.to(dt).contiguous()
-    w = weight.to(dt).contiguous()
+    q, w = _lib.as_type(query, dt), _lib.as_type(weight, dt)
     out = torch.empty(B, T, D, dtype=dt, device=x0.device)
     n = len(srcs)
     ptrs = (ctypes.c_void_p * n)(*[s.data_ptr() for s in srcs])
@@ -102,9 +101,8 @@ def attn_res_read_norms(sources, query, norm, norm_a, norm_b):
             raise ValueError('attn_res_read_norms: sources must share shape and dtype')
     dev = x0.device
     weight = norm.weight if norm.weight is not None else torch.ones(D, dtype=dt, device=dev)
-    q = query.to(dt).contiguous()
-    w = weight.to(dt).contiguous()
-    wa, wb = norm_a.weight.to(dt).contiguous(), norm_b.weight.to(dt).contiguous()
+    q, w = _lib.as_type(query, dt), _lib.as_type(weight, dt)
+    wa, wb = _lib.as_type(norm_a.weight, dt), _lib.as_type(norm_b.weight, dt)
     ya = torch.empty(B, T, D, dtype=dt, device=dev)
     yb = torch.empty(B, T, D, dtype=dt, device=dev)
     n = len(srcs)

@@ -341,8 +341,10 @@ def gdn_prefill_fused(proj, offsets, conv_weights, tails, a_log, dt_bias, q_scal
     H = heads
     dev = proj.device
     C = (H * dk, H * dk, H * dv)
-    ws_ = [w.detach().reshape(c, 4).to(torch.bfloat16).contiguous() for w, c in zip(conv_weights, C)]
-    tin = [None if t is None else t.detach().to(torch.bfloat16).contiguous() for t in tails]
+    if any(w.numel() != 4 * c for w, c in zip(conv_weights, C)):
+        raise ValueError('gdn_prefill_fused: conv weights must be [H * dk, 1, 4] (q, k) and [H * dv, 1, 4] (v)')
+    ws_ = [_lib.as_type(w, torch.bfloat16) for w in conv_weights]
+    tin = [None if t is None else _lib.as_type(t, torch.bfloat16) for t in tails]
     if any(t is not None for t in tin) and (cu_seqlens is not None or not all(t is not None for t in tin)):
         return None
     if cu_seqlens is None:
@@ -367,9 +369,7 @@ def gdn_prefill_fused(proj, offsets, conv_weights, tails, a_log, dt_bias, q_scal
     tout = [torch.empty(nseq, c, 3, dtype=torch.bfloat16, device=dev) for c in C]
     nbytes = _lib.lib().motif_gdn_chunk_workspace_bytes(H, dk, dv, 64, max(total, 1))
     ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=dev)
-    al = a_log.detach().to(torch.bfloat16).contiguous()
-    db = dt_bias.detach().to(torch.bfloat16).contiguous()
-    nw = norm_weight.detach().to(torch.bfloat16).contiguous()
+    al, db, nw = (_lib.as_type(t, torch.bfloat16) for t in (a_log, dt_bias, norm_weight))
     rc = _lib.lib().motif_gdn_prefill_fused(
         proj.data_ptr(), proj.stride(0), proj.stride(1), *[int(o) for o in offsets],
         ws_[0].data_ptr(), ws_[1].data_ptr(), ws_[2].data_ptr(), 4,

@@ -31,7 +31,9 @@ def gdn_decode_fused(proj, offsets, conv_weights, tails, a_log, dt_bias, norm_we
     if proj.stride(-1) != 1:
         proj = proj.contiguous()
     K = conv_weights[0].shape[-1]
-    ws = [w.detach().reshape(w.shape[0], K).to(dt).contiguous() for w in conv_weights]
+    if any(w.numel() != w.shape[0] * K for w in conv_weights):
+        raise ValueError(f'gdn_decode_fused: conv weights must be [C, 1, {K}]')
+    ws = [_lib.as_type(w, dt) for w in conv_weights]
     for t in tails:
         if t.dtype != dt or not t.is_contiguous():
             raise ValueError('gdn_decode_fused: conv tails must be contiguous and in the activation dtype')
@@ -43,9 +45,7 @@ def gdn_decode_fused(proj, offsets, conv_weights, tails, a_log, dt_bias, norm_we
     for t in (state, state_out):
         if t.dtype != torch.float32 or not t.is_contiguous() or t.shape != (B, H, dk, dv):
             raise ValueError('gdn_decode_fused: state must be contiguous fp32 [B, H, dk, dv]')
-    al = a_log.detach().to(dt).contiguous()
-    db = dt_bias.detach().to(dt).contiguous()
-    nw = norm_weight.detach().to(dt).contiguous()
+    al, db, nw = _lib.as_type(a_log, dt), _lib.as_type(dt_bias, dt), _lib.as_type(norm_weight, dt)
     y = torch.empty(B, H * dv, dtype=dt, device=proj.device)
     rc = _lib.lib().motif_gdn_decode_fused(
         proj.data_ptr(), proj.stride(0), *[int(o) for o in offsets],

@@ -45,6 +45,8 @@ def rows_eligible(x, weight, bias=None):
     M = x.numel() // K if K else 0
     if M == 0 or M > MAX_ROWS:
         return False
+    if x.is_contiguous():  # rows of K elements, K % 32 == 0: only the addresses are left to check
+        return x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
     x2, _ = _rows2d(x)
     if x2 is None or x2.stride(0) % 8 or x2.data_ptr() % 16 or weight.data_ptr() % 16:
         return False
@@ -65,6 +67,14 @@ def linear_rows(x, weight, epilogue='none', aux=None, aux2=None, out=None, out2=
     code = EPILOGUES[epilogue]
     if wants_grad(x, weight, aux, aux2):
         return _torch_form(x, weight, code, aux, aux2)
+    if code == 0 and out is None and x.is_contiguous():  # (no views to build)
+        K, N = x.shape[-1], weight.shape[0]
+        y = torch.empty(*x.shape[:-1], N, dtype=x.dtype, device=x.device)
+        rc = _lib.lib().motif_linear_rows(x.data_ptr(), K, weight.data_ptr(), weight.stride(0), y.data_ptr(), N,
+                                          x.numel() // K if K else 0, N, K, 0, None, 0, None, 0, None, 0,
+                                          _lib.stream_ptr(x.device))
+        _lib.check(rc, 'motif_linear_rows')
+        return y
     x2, lead = _rows2d(x)
     if x2 is None:
         x2 = x.reshape(-1, x.shape[-1]).contiguous()
