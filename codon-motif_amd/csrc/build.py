@@ -28,12 +28,13 @@ FLAGS = [
     '-Xclang', '-target-feature', '-Xclang', '-packed-fp32-ops',
     '-I', os.path.join(os.path.dirname(os.path.dirname(HERE)), 'include'),
 ]
-# Per-source extras.  chord.hip and gdn_chunk.hip: MFMA accumulators in ordinary VGPRs,
-# so the softmax / rescale code and the scan's per-chunk chain read them without
-# accumulator-register copies.  The backward kernels keep the default: their register
-# budgets rely on the accumulator file (the VGPR form made the per-chunk gradient
-# kernel 19% slower).
-EXTRA = {'chord.hip': ['-mllvm', '-amdgpu-mfma-vgpr-form'], 'gdn_chunk.hip': ['-mllvm', '-amdgpu-mfma-vgpr-form']}
+# Per-source extras: MFMA accumulators in ordinary VGPRs, so the softmax / rescale code and
+# the scan's per-chunk chain read them without accumulator-register copies (the dQ kernel of
+# chord_bwd.hip spent 100 of 520 instructions per tile on them).  The GDN backward kernels keep
+# the default: their register budgets rely on the accumulator file (the VGPR form made the
+# per-chunk gradient kernel of gdn_bwd_chunk.hip 19% slower).
+_VGPR_FORM = ['-mllvm', '-amdgpu-mfma-vgpr-form']
+EXTRA = {f: _VGPR_FORM for f in ('chord.hip', 'chord_bwd.hip', 'gdn_chunk.hip')}
 
 
 def _run(cmd, verbose):

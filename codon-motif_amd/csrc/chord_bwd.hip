@@ -21,12 +21,19 @@
 // dV^T += dO^T P, dK^T += Q^T (s c dZ).
 // The causal loop of a block is cut into chunks of at most `cq` / `ckv` tiles so that no
 // workgroup runs much longer than the average (the heaviest block otherwise sets the
-// kernel's length); chunks write fp32 partials that chord_bwd_reduce_*_kernel sum in a
+// kernel's length); chunks write fp32 partials that chord_bwd_reduce_kernel sums in a
 // fixed order (with one chunk and no GQA sharing the kernels write bf16 directly).
 // Both loops keep two LDS tile buffers (one barrier per tile) and the next tile's global
 // loads in registers.  The GGD bias (and, in the dQ kernel, its three parameter
 // derivatives) come from per-wave windows over the 63 distances a 32 x 32 tile meets,
 // evaluated in registers; tiles wholly below the causal diagonal skip the masks.
+//
+// Bound by VALU issue (a tile's 1024 scores take ~10 instructions each and one exp2, its 12 or 16
+// MFMAs a third of that), so what is not per score is kept off the vector unit: tiles come through
+// range-checked buffers with fixed lane offsets, accumulators sit in ordinary registers, dQ's column
+// factor c s is taken after the sum, the dK / dV kernel reads a query's four values as one row that
+// the dQ kernel wrote.  B = 2, 12 heads, 2048 tokens: dQ 74 -> 57 us, dK / dV 73 -> 62, reductions
+// 25 (three launches) -> 13 (one).
 #include <algorithm>
 #include <string>
 
@@ -57,7 +64,7 @@ struct ChordBwdArgs {
   bf16_t *dv; int64_t dv_sb, dv_sh, dv_st;
   float *dparam;  // [4][H]: d alpha, d beta, d mu, d ssmax
   // workspace
-  float *delta;   // [B][H][L]
+  float4 *rows;   // [B][H][L]: {log-sum-exp, Delta, c log2(e), c s} of a query
   float *pparam;  // [nsq][B][nqb][H][4] parameter partial sums
   float *pq;      // [nsq][B][H][L][64] dQ partials (nsq > 1)
   float *pk, *pv; // [nskv][H][B][S][64] dK / dV partials (unless kv_direct)
@@ -92,15 +99,25 @@ __device__ __forceinline__ bf16x8 pack8(const float *x) {
 __device__ __forceinline__ uint4 ld16(const bf16_t *p) { return *reinterpret_cast<const uint4 *>(p); }
 
 // Tile staging by 128 threads t: rows 2 (t & 15) and + 1, 8-element segment t >> 4 of a
-// 32-row x 64 tile of [rows][64] bf16 rows (row r at base + r * st); rows at or past
-// `nrows` read 0.  The loads go to registers one tile ahead of the stores.
+// 32-row x 64 tile of [rows][64] bf16 rows, through a range-checked buffer that starts at the
+// tile's first row (uniform) and ends at row `nrows` of the matrix: rows past it read 0 with no
+// branch, and a tile costs two loads and its base.  The loads go to registers one tile ahead of the
+// stores.
 struct Stage2 { uint4 a, b; };
-__device__ __forceinline__ Stage2 stage_load(const bf16_t *base, int64_t st, int nrows, int t) {
-  const int pr = t & 15, seg = t >> 4;
-  const int r0 = 2 * pr, r1 = 2 * pr + 1;
-  const uint4 z = {0u, 0u, 0u, 0u};
-  return {r0 < nrows ? ld16(base + r0 * st + 8 * seg) : z, r1 < nrows ? ld16(base + r1 * st + 8 * seg) : z};
-}
+struct StageSrc {
+  const bf16_t *base;
+  int64_t st;
+  int nrows;
+  uint32_t off, off1;  // this thread's two row segments
+  __device__ __forceinline__ StageSrc(const bf16_t *p, int64_t s, int n, int t)
+      : base(p), st(s), nrows(n), off(static_cast<uint32_t>((2 * (t & 15) * s + 8 * (t >> 4)) * 2)),
+        off1(off + static_cast<uint32_t>(2 * s)) {}
+  __device__ __forceinline__ Stage2 load(int row0) const {
+    const int rows = min(kT, nrows - row0);
+    const buf_t buf = make_buf(base + int64_t(row0) * st, rows > 0 ? static_cast<uint32_t>(((rows - 1) * st + kBD) * 2) : 0u);
+    return {buf_ld16(buf, off), buf_ld16(buf, off1)};
+  }
+};
 // The rows (padded) into `rows`, and, when `tr` is set, the transposed tile [64][32]
 // (elements in tperm order) into `tr`.
 __device__ __forceinline__ void stage_store(const Stage2 &g, int t, bf16_t *rows, bf16_t *tr) {
@@ -133,6 +150,12 @@ __global__ void __launch_bounds__(256) chord_bwd_dq_kernel(ChordBwdArgs a) {
   const int q0 = qb * kBlk + 32 * w;
   const int my_q = q0 + lc;
   const bool qv = my_q < a.L;
+  const int kv_end = min(a.S, a.q_start + min(a.L, qb * kBlk + kBlk));
+  // waves 0, 1 stage K (rows and K^T), 2, 3 V (rows); the first tile's loads go ahead of the rest
+  const bool kside = w < 2;
+  const StageSrc src(kside ? a.k + b * a.k_sb + kvh * a.k_sh : a.v + b * a.v_sb + kvh * a.v_sh, kside ? a.k_st : a.v_st,
+                     kv_end, tid & 127);
+  Stage2 stg = src.load(t_begin * kT);
   const int qr = min(my_q, a.L - 1);
 
   // this lane's query row: Q and dO as B operands (d = 16 ds + 8 hh .. +8), Delta
@@ -155,14 +178,13 @@ __global__ void __launch_bounds__(256) chord_bwd_dq_kernel(ChordBwdArgs a) {
   }
   const float delta = dsum;
   const size_t ri = (static_cast<size_t>(b) * a.H + h) * a.L + my_q;
-  if (chunk == 0 && qv && hh == 0) a.delta[ri] = delta;
   const float lse2 = qv ? a.lse[ri] : 0.f;
   const float lam = a.log_n[b * a.ln_sb + int64_t(qr) * a.ln_st];
   const float sig = a.ssmax[h], al = a.alpha[h], be = a.beta[h], mu = a.mu[h];
   const float s = a.scale, c = sig * lam, cl = c * kLog2e, cs = c * s;
+  if (chunk == 0 && qv && hh == 0) a.rows[ri] = float4{lse2, delta, cl, cs};
   const int q_abs = a.q_start + my_q;
   const int wave_kv_end = a.q_start + min(a.L, q0 + 32);  // keys this wave sees: < wave_kv_end
-  const int kv_end = min(a.S, a.q_start + min(a.L, qb * kBlk + kBlk));
 
   __shared__ __attribute__((aligned(16))) bf16_t sK[2][kT * kRowP];    // K rows of the tile
   __shared__ __attribute__((aligned(16))) bf16_t sV[2][kT * kRowP];    // V rows
@@ -170,31 +192,21 @@ __global__ void __launch_bounds__(256) chord_bwd_dq_kernel(ChordBwdArgs a) {
   __shared__ float4 sW[4][64];  // per wave: {b, d/d alpha, d/d beta, d/d mu} per distance
   __shared__ float sRed[4][4];
 
-  const bf16_t *kbase = a.k + b * a.k_sb + kvh * a.k_sh;
-  const bf16_t *vbase = a.v + b * a.v_sb + kvh * a.v_sh;
   f32x16 dqacc[2];
   dqacc[0] = f32x16{};
   dqacc[1] = f32x16{};
   float sa = 0.f, sb = 0.f, sm = 0.f, ss = 0.f;
 
-  // threads 0-127 stage K (rows and K^T), 128-255 V (rows)
-  const bool kside = tid < 128;
-  const int st_t = tid & 127;
-  auto load_kv = [&](int n0) {
-    return kside ? stage_load(kbase + int64_t(n0) * a.k_st, a.k_st, kv_end - n0, st_t)
-                 : stage_load(vbase + int64_t(n0) * a.v_st, a.v_st, kv_end - n0, st_t);
-  };
-  auto store_kv = [&](const Stage2 &g, int buf) { stage_store(g, st_t, kside ? sK[buf] : sV[buf], kside ? sKT[buf] : nullptr); };
-  Stage2 stg = load_kv(t_begin * kT);
+  auto store_kv = [&](const Stage2 &g, int buf) { stage_store(g, tid & 127, kside ? sK[buf] : sV[buf], kside ? sKT[buf] : nullptr); };
   store_kv(stg, 0);
-  if (t_begin + 1 < t_end) stg = load_kv((t_begin + 1) * kT);
+  stg = src.load((t_begin + 1) * kT);  // (past the last tile: zeros)
   __syncthreads();
 
   for (int kt = t_begin; kt < t_end; ++kt) {
     const int n0 = kt * kT, buf = (kt - t_begin) & 1;
     if (kt + 1 < t_end) {  // the next tile into the other buffer (free since the last barrier)
       store_kv(stg, buf ^ 1);
-      if (kt + 2 < t_end) stg = load_kv(n0 + 2 * kT);
+      stg = src.load(n0 + 2 * kT);
     }
     if (n0 < wave_kv_end) {
       // window entry j (lane j < 63): distance d = key - q_abs = n0 - q_start - q0 - 31 + j
@@ -229,12 +241,12 @@ __global__ void __launch_bounds__(256) chord_bwd_dq_kernel(ChordBwdArgs a) {
           const float rr = fmaf(s, sacc[r], wv.x);
           float p = fast_exp2(fmaf(cl, rr, -lse2));
           if constexpr (decltype(masked)::value) p = (qv && n0 + kk <= q_abs) ? p : 0.f;
-          const float g = p * (pacc[r] - delta);
+          const float g = p * (pacc[r] - delta);  // (dQ's factor c s is the column's: taken at the end)
           ss = fmaf(g, rr, ss);
           sa = fmaf(g, wv.y, sa);
           sb = fmaf(g, wv.z, sb);
           sm = fmaf(g, wv.w, sm);
-          dz[r] = g * cs;
+          dz[r] = g;
         }
       };
       // every key of the tile at or before every query of the wave, all queries valid
@@ -253,6 +265,11 @@ __global__ void __launch_bounds__(256) chord_bwd_dq_kernel(ChordBwdArgs a) {
     __syncthreads();  // this tile's reads done, the next tile's stores visible
   }
 
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    dqacc[0][r] *= cs;
+    dqacc[1][r] *= cs;
+  }
   if (qv) {
     if (a.nsq == 1) {
       bf16_t *dst = a.dq + b * a.dq_sb + h * a.dq_sh + int64_t(my_q) * a.dq_st;
@@ -300,6 +317,18 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
   const int k0w = kb * kBlk + 32 * w;
   const int my_k = k0w + lc;
   const bool kvld = my_k < a.S;
+  // waves 0, 1 stage Q, 2, 3 dO (rows and transposed); threads 0-31 the row values; the first
+  // tile's loads go ahead of the rest
+  const bool qside = w < 2;
+  const size_t rbase = (static_cast<size_t>(b) * a.H + h) * a.L;
+  const StageSrc src(qside ? a.q + b * a.q_sb + h * a.q_sh : a.dout + b * a.d_sb + h * a.d_sh, qside ? a.q_st : a.d_st, a.L,
+                     tid & 127);
+  auto load_row = [&](int i0) {  // (queries past L: zeros, c = 0)
+    const int n = min(kT, a.L - i0);
+    return __builtin_bit_cast(float4, buf_ld16(make_buf(a.rows + rbase + i0, n > 0 ? n * 16u : 0u), 16u * (tid & (kT - 1))));
+  };
+  Stage2 stg = src.load(t_begin * kT);
+  float4 rowv = load_row(t_begin * kT);
   const int kr = min(my_k, a.S - 1);
 
   const bf16_t *krow = a.k + b * a.k_sb + kvh * a.k_sh + int64_t(kr) * a.k_st;
@@ -322,49 +351,21 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
   dkacc[0] = dkacc[1] = dvacc[0] = dvacc[1] = f32x16{};
   const float s = a.scale;
   const float sig = a.ssmax[h], al = a.alpha[h], be = a.beta[h], mu = a.mu[h];
-  const bf16_t *qbase = a.q + b * a.q_sb + h * a.q_sh;
-  const bf16_t *dbase = a.dout + b * a.d_sb + h * a.d_sh;
-  const size_t rbase = (static_cast<size_t>(b) * a.H + h) * a.L;
-
-  // threads 0-127 stage Q, 128-255 dO (rows and transposed); threads 0-31 the row values
-  const bool qside = tid < 128;
-  const int st_t = tid & 127;
-  auto load_q = [&](int i0) {
-    return qside ? stage_load(qbase + int64_t(i0) * a.q_st, a.q_st, a.L - i0, st_t)
-                 : stage_load(dbase + int64_t(i0) * a.d_st, a.d_st, a.L - i0, st_t);
-  };
-  auto load_row = [&](int i0) {
-    const int i = i0 + (tid & (kT - 1));
-    const bool iv = i < a.L;
-    const size_t ri = rbase + (iv ? i : 0);
-    const float c = iv ? sig * a.log_n[b * a.ln_sb + int64_t(i) * a.ln_st] : 0.f;
-    return float4{iv ? a.lse[ri] : 0.f, iv ? a.delta[ri] : 0.f, c * kLog2e, c * s};
-  };
   auto store_q = [&](const Stage2 &g, const float4 &rv, int buf) {
-    stage_store(g, st_t, qside ? sQ[buf] : sD[buf], qside ? sQT[buf] : sDT[buf]);
+    stage_store(g, tid & 127, qside ? sQ[buf] : sD[buf], qside ? sQT[buf] : sDT[buf]);
     if (tid < kT) sRow[buf][tid] = rv;
   };
-  Stage2 stg = {};
-  float4 rowv = {};
-  if (t_begin < t_end) {
-    stg = load_q(t_begin * kT);
-    if (tid < kT) rowv = load_row(t_begin * kT);
-    store_q(stg, rowv, 0);
-    if (t_begin + 1 < t_end) {
-      stg = load_q((t_begin + 1) * kT);
-      if (tid < kT) rowv = load_row((t_begin + 1) * kT);
-    }
-  }
+  store_q(stg, rowv, 0);
+  stg = src.load((t_begin + 1) * kT);
+  rowv = load_row((t_begin + 1) * kT);
   __syncthreads();
 
   for (int qt = t_begin; qt < t_end; ++qt) {
     const int i0 = qt * kT, buf = (qt - t_begin) & 1;
     if (qt + 1 < t_end) {  // the next tile into the other buffer (free since the last barrier)
       store_q(stg, rowv, buf ^ 1);
-      if (qt + 2 < t_end) {
-        stg = load_q(i0 + 2 * kT);
-        if (tid < kT) rowv = load_row(i0 + 2 * kT);
-      }
+      stg = src.load(i0 + 2 * kT);
+      rowv = load_row(i0 + 2 * kT);
     }
     // a wave whose keys all lie past the tile's last query (or past S) skips it
     if (k0w < a.S && a.q_start + i0 + kT - 1 >= k0w) {
@@ -386,6 +387,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
         pacc = mma32(dov, vreg[ds], pacc);
       }
       float pv[16], dz[16];
+      // the tile's queries that see this lane's key: q_lo .. q_lo + q_n - 1 (one compare per element)
+      const int q_lo = max(0, my_k - a.q_start - i0);
+      const uint32_t q_n = kvld ? max(0, min(kT, a.L - i0) - q_lo) : 0;
       auto body = [&](auto masked) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
@@ -393,7 +397,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
           const float4 rw = sRow[buf][qq];
           const float rr = fmaf(s, sacc[r], sW[w][lc - qq + 31]);
           float p = fast_exp2(fmaf(rw.z, rr, -rw.x));
-          if constexpr (decltype(masked)::value) p = (kvld && i0 + qq < a.L && my_k <= a.q_start + i0 + qq) ? p : 0.f;
+          if constexpr (decltype(masked)::value) p = static_cast<uint32_t>(qq - q_lo) < q_n ? p : 0.f;
           pv[r] = p;
           dz[r] = p * (pacc[r] - rw.y) * rw.w;
         }
@@ -447,9 +451,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 
 // dK / dV of kv head kvh = the sum over its GQA group's query heads and the chunks of the
 // key's block, in that order, rounded to bf16; one thread per 4 elements.
-__global__ void __launch_bounds__(256) chord_bwd_reduce_kv_kernel(ChordBwdArgs a) {
+__device__ __forceinline__ void reduce_kv(const ChordBwdArgs &a, int block) {
   const int64_t n4 = static_cast<int64_t>(a.B) * a.Hkv * a.S * (kBD / 4);
-  const int64_t e = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  const int64_t e = static_cast<int64_t>(block) * 256 + threadIdx.x;
   if (e >= n4) return;
   const int d0 = 4 * static_cast<int>(e % (kBD / 4));
   const int64_t rest = e / (kBD / 4);
@@ -477,9 +481,9 @@ __global__ void __launch_bounds__(256) chord_bwd_reduce_kv_kernel(ChordBwdArgs a
 }
 
 // dQ = the sum over the chunks of the query's block, in order, rounded to bf16.
-__global__ void __launch_bounds__(256) chord_bwd_reduce_q_kernel(ChordBwdArgs a) {
+__device__ __forceinline__ void reduce_q(const ChordBwdArgs &a, int block) {
   const int64_t n4 = static_cast<int64_t>(a.B) * a.H * a.L * (kBD / 4);
-  const int64_t e = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  const int64_t e = static_cast<int64_t>(block) * 256 + threadIdx.x;
   if (e >= n4) return;
   const int d0 = 4 * static_cast<int>(e % (kBD / 4));
   const int64_t rest = e / (kBD / 4);
@@ -499,8 +503,8 @@ __global__ void __launch_bounds__(256) chord_bwd_reduce_q_kernel(ChordBwdArgs a)
 
 // dparam[k][h] = the sum of the dQ workgroups' partials (batch rows, query blocks, chunks):
 // one wave per (k, h), lanes over (batch row, query block) in a fixed order.
-__global__ void __launch_bounds__(64) chord_bwd_reduce_param_kernel(ChordBwdArgs a) {
-  const int t = blockIdx.x, h = t % a.H, k = t / a.H, lane = threadIdx.x;
+__device__ __forceinline__ void reduce_param(const ChordBwdArgs &a, int t) {
+  const int h = t % a.H, k = t / a.H, lane = threadIdx.x & 63;
   float acc = 0.f;
   for (int e = lane; e < a.B * a.nqb; e += 64) {
     const int b = e / a.nqb, qb = e - b * a.nqb;
@@ -511,10 +515,24 @@ __global__ void __launch_bounds__(64) chord_bwd_reduce_param_kernel(ChordBwdArgs
   if (lane == 0) a.dparam[k * a.H + h] = acc;
 }
 
+// Every reduction in one launch (three apart took 12.5 + 7.7 + 4.7 us at B = 2, 12 heads, 2048
+// tokens, most of it launch and tail): workgroups [0, nkv) dK / dV, then nq of dQ, then one of four
+// waves per four parameter sums.
+__global__ void __launch_bounds__(256) chord_bwd_reduce_kernel(ChordBwdArgs a, int nkv, int nq) {
+  const int block = blockIdx.x;
+  if (block < nkv) return reduce_kv(a, block);
+  if (block < nkv + nq) return reduce_q(a, block - nkv);
+  const int t = 4 * (block - nkv - nq) + (threadIdx.x >> 6);
+  if (t < 4 * a.H) reduce_param(a, t);
+}
+
 }  // namespace
 
-// Chunk sizes: about 1024 chunks over the whole causal loop, at least 16 tiles each and at
-// most 8 chunks per block.
+// Chunk sizes: about as many full chunks over the whole causal loop as the kernel's workgroups fit
+// on the chip at once (dQ: three per CU, dK / dV: two; blocks end in shorter chunks, so the counts
+// aimed at lie below 768 and 512), at least 6 tiles each and at most 8 chunks per block.  Swept at
+// 12 heads (whole backward, us; 1024 chunks of at least 16 tiles before): 2 x 2048 tokens 141 ->
+// 117, 4096 tokens (3 kv heads) 209 -> 186, 1024 tokens 57 -> 47, 700 tokens 57 -> 42.
 struct BwdPlan {
   int nqb, nkb, cq, nsq, ckv, nskv;
   bool kv_direct;
@@ -525,19 +543,19 @@ static BwdPlan plan_bwd(int B, int H, int Hkv, int L, int S, int q_start) {
   BwdPlan p{};
   p.nqb = (L + kBlk - 1) / kBlk;
   p.nkb = (S + kBlk - 1) / kBlk;
-  auto chunking = [](int64_t total, int maxt, int &csize, int &ns) {
-    csize = static_cast<int>(std::max<int64_t>({16, (total + 1023) / 1024, (maxt + 7) / 8}));
+  auto chunking = [](int64_t total, int maxt, int target, int &csize, int &ns) {
+    csize = static_cast<int>(std::max<int64_t>({6, (total + target - 1) / target, (maxt + 7) / 8}));
     ns = std::max(1, (maxt + csize - 1) / csize);
   };
   int64_t tq = 0, tkv = 0;
   for (int qb = 0; qb < p.nqb; ++qb) tq += dq_tiles(qb, L, q_start);
   const int qt_end = (L + kT - 1) / kT;
   for (int kb = 0; kb < p.nkb; ++kb) tkv += std::max(0, qt_end - kv_first_tile(kb, q_start));
-  chunking(tq * B * H, p.nqb ? dq_tiles(p.nqb - 1, L, q_start) : 0, p.cq, p.nsq);
-  chunking(tkv * B * H, qt_end, p.ckv, p.nskv);
+  chunking(tq * B * H, p.nqb ? dq_tiles(p.nqb - 1, L, q_start) : 0, 640, p.cq, p.nsq);
+  chunking(tkv * B * H, qt_end, 384, p.ckv, p.nskv);
   p.kv_direct = H == Hkv && p.nskv == 1;
   auto al = [](size_t x) { return (x + 255) / 256 * 256; };
-  size_t off = al(static_cast<size_t>(B) * H * L * sizeof(float));  // Delta
+  size_t off = al(static_cast<size_t>(B) * H * L * sizeof(float4));  // the query rows' values
   p.off_param = off;
   off += al(static_cast<size_t>(p.nsq) * B * p.nqb * H * 4 * sizeof(float));
   p.off_pq = off;
@@ -586,8 +604,8 @@ extern "C" int motif_chord_bwd(
     z.H = H;
     z.cq = 1;
     z.dparam = dparam;
-    chord_bwd_reduce_param_kernel<<<dim3(4 * H), dim3(64), 0, s>>>(z);
-    return check_launch("chord_bwd_reduce_param_kernel");
+    chord_bwd_reduce_kernel<<<dim3(H), dim3(256), 0, s>>>(z, 0, 0);
+    return check_launch("chord_bwd_reduce_kernel");
   }
   if (!q || !k || !v || !out || !dout || !lse || !alpha || !beta || !mu || !ssmax || !log_n || !dq || !dk || !dv)
     return set_error(MOTIF_ERR_INVALID, "chord_bwd: NULL pointer");
@@ -596,10 +614,13 @@ extern "C" int motif_chord_bwd(
   const uintptr_t al = reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v) |
                        reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(dout) |
                        reinterpret_cast<uintptr_t>(dq) | reinterpret_cast<uintptr_t>(dk) | reinterpret_cast<uintptr_t>(dv);
+  // (32-bit offsets inside a 32-row tile)
+  for (int64_t x : {q_st, k_st, v_st, d_st})
+    if (x < 0 || x >= (int64_t(1) << 25)) return set_error(MOTIF_ERR_UNSUPPORTED, "chord_bwd: row stride out of range");
   if ((st & 7) != 0 || (al & 15) != 0) return set_error(MOTIF_ERR_UNSUPPORTED, "chord_bwd: need 16-byte aligned rows");
   const BwdPlan pl = plan_bwd(B, H, Hkv, L, S, q_start);
-  if (!workspace || workspace_bytes < pl.bytes)
-    return set_error(MOTIF_ERR_INVALID, "chord_bwd: workspace too small (need " + std::to_string(pl.bytes) + " bytes)");
+  if (!workspace || workspace_bytes < pl.bytes || (reinterpret_cast<uintptr_t>(workspace) & 15))
+    return set_error(MOTIF_ERR_INVALID, "chord_bwd: workspace too small or not 16-byte aligned (need " + std::to_string(pl.bytes) + " bytes)");
   ChordBwdArgs a;
   a.q = static_cast<const bf16_t *>(q); a.q_sb = q_sb; a.q_sh = q_sh; a.q_st = q_st;
   a.k = static_cast<const bf16_t *>(k); a.k_sb = k_sb; a.k_sh = k_sh; a.k_st = k_st;
@@ -613,7 +634,7 @@ extern "C" int motif_chord_bwd(
   a.dv = static_cast<bf16_t *>(dv); a.dv_sb = dv_sb; a.dv_sh = dv_sh; a.dv_st = dv_st;
   a.dparam = dparam;
   char *ws = static_cast<char *>(workspace);
-  a.delta = reinterpret_cast<float *>(ws);
+  a.rows = reinterpret_cast<float4 *>(ws);
   a.pparam = reinterpret_cast<float *>(ws + pl.off_param);
   a.pq = reinterpret_cast<float *>(ws + pl.off_pq);
   a.pk = reinterpret_cast<float *>(ws + pl.off_pk);
@@ -626,20 +647,13 @@ extern "C" int motif_chord_bwd(
   if (L > 0) {  // with no queries dK and dV are zero (the dK / dV pass below writes them)
     chord_bwd_dq_kernel<<<dim3(H, pl.nqb, B * pl.nsq), dim3(256), 0, s>>>(a);
     if ((rc = check_launch("chord_bwd_dq_kernel"))) return rc;
-    if (pl.nsq > 1) {
-      const int64_t n4 = static_cast<int64_t>(B) * H * L * (kBD / 4);
-      chord_bwd_reduce_q_kernel<<<dim3(static_cast<unsigned>((n4 + 255) / 256)), dim3(256), 0, s>>>(a);
-      if ((rc = check_launch("chord_bwd_reduce_q_kernel"))) return rc;
-    }
   }
-  chord_bwd_reduce_param_kernel<<<dim3(4 * H), dim3(64), 0, s>>>(a);
-  if ((rc = check_launch("chord_bwd_reduce_param_kernel"))) return rc;
   chord_bwd_dkdv_kernel<<<dim3(H, pl.nkb, B * pl.nskv), dim3(256), 0, s>>>(a);
   if ((rc = check_launch("chord_bwd_dkdv_kernel"))) return rc;
-  if (!pl.kv_direct) {
-    const int64_t n4 = static_cast<int64_t>(B) * Hkv * S * (kBD / 4);
-    chord_bwd_reduce_kv_kernel<<<dim3(static_cast<unsigned>((n4 + 255) / 256)), dim3(256), 0, s>>>(a);
-    if ((rc = check_launch("chord_bwd_reduce_kv_kernel"))) return rc;
-  }
+  auto blocks = [](int64_t rows) { return static_cast<int>((rows * (kBD / 4) + 255) / 256); };
+  const int nkv = pl.kv_direct ? 0 : blocks(static_cast<int64_t>(B) * Hkv * S);
+  const int nq = L > 0 && pl.nsq > 1 ? blocks(static_cast<int64_t>(B) * H * L) : 0;
+  chord_bwd_reduce_kernel<<<dim3(nkv + nq + H), dim3(256), 0, s>>>(a, nkv, nq);
+  if ((rc = check_launch("chord_bwd_reduce_kernel"))) return rc;
   return MOTIF_OK;
 }
