@@ -606,7 +606,11 @@ extern "C" int motif_gdn_chunk_bwd(
   if (dk != kDK || (dv != 64 && dv != 128))
     return set_error(MOTIF_ERR_UNSUPPORTED, "gdn_chunk_bwd: needs dk == 64 and dv in {64, 128}");
   if (dtype != MOTIF_F32 && dtype != MOTIF_BF16) return set_error(MOTIF_ERR_UNSUPPORTED, "gdn_chunk_bwd: unsupported dtype");
-  if (B == 0 || H == 0 || L == 0) return MOTIF_OK;
+  if (B == 0 || H == 0) return MOTIF_OK;
+  if (L == 0) {  // (no step to go through: the state's gradient is the final state's)
+    if (!dstate_in) return set_error(MOTIF_ERR_INVALID, "gdn_chunk_bwd: NULL pointer");
+    return motif_gdn_opscan_f32(nullptr, nullptr, dstate_out, nullptr, dstate_in, B * H, 0, dk, dv, 1, 0, stream);
+  }
   if (!q || !k || !v || !beta || !g || !dout || !dq || !dk_ || !dv_ || !dbeta || !dg || !dstate_in)
     return set_error(MOTIF_ERR_INVALID, "gdn_chunk_bwd: NULL pointer");
   const int N = (L + kC - 1) / kC;

@@ -91,3 +91,15 @@ def test_mixed_types():
     for a, r, t in zip(got, ref, ts):
         assert a.dtype == t.dtype
         assert ((a.double().cpu() - r).norm() / r.norm()).item() < _bar(x) + 2 ** -8
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16])
+def test_empty_sequence_passes_the_state_gradient(dtype):
+    x, S0, do, dS = _case(2, 3, 0, 64, dtype)
+    ts = [t.to(DEV).requires_grad_() for t in x]
+    s0 = S0.to(DEV).requires_grad_()
+    o, S = chunk_gated_delta_rule(*ts, s0)
+    assert o.shape == do.shape and torch.equal(S, s0)
+    got = torch.autograd.grad([o, S], [*ts, s0], [do.to(DEV), dS.to(DEV)])
+    assert all(a.shape == t.shape for a, t in zip(got, [*ts, s0]))
+    assert torch.equal(got[-1].cpu(), dS)
