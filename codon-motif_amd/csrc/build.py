@@ -30,11 +30,11 @@ FLAGS = [
 ]
 # Per-source extras: MFMA accumulators in ordinary VGPRs, so the softmax / rescale code and
 # the scan's per-chunk chain read them without accumulator-register copies (the dQ kernel of
-# chord_bwd.hip spent 100 of 520 instructions per tile on them).  The GDN backward kernels keep
+# chord_bwd.hip spent 100 of 520 instructions per tile on them).  The per-chunk GDN backward kernels keep
 # the default: their register budgets rely on the accumulator file (the VGPR form made the
 # per-chunk gradient kernel of gdn_bwd_chunk.hip 19% slower).
 _VGPR_FORM = ['-mllvm', '-amdgpu-mfma-vgpr-form']
-EXTRA = {f: _VGPR_FORM for f in ('chord.hip', 'chord_bwd.hip', 'gdn_chunk.hip')}
+EXTRA = {f: _VGPR_FORM for f in ('chord.hip', 'chord_bwd.hip', 'gdn_bwd.hip', 'gdn_chunk.hip')}
 
 
 def _run(cmd, verbose):

@@ -256,22 +256,34 @@ int launch_scan(const ScanArgs &a, int BH, hipStream_t stream) {
 // all chunks in parallel.  The kernel walks S <- M_n S + Q_n over the chunks in order
 // (REV: last to first) and records S before each step: P_n (forward) or dSn_n (reverse),
 // with M = A (forward) or A^T (reverse) handed in row-major.
-// Workgroup = (16 state columns, batch.head), 4 waves; wave w owns state row tiles
-// w, w + 4, ...  M_n goes through LDS (double buffered, filled from registers loaded
-// kOpDepth chunks ahead), S^T through LDS (double buffered) for the B operands; the k-sum
-// of each tile is split over four accumulators (independent MFMA chains).  TRANS reads
-// M_n transposed (the reverse scan takes A_n as the forward scan does).  Workgroups go
-// to the 8 XCDs round-robin by linear id: the column groups of one batch.head are
-// placed on one XCD, so each M_n comes from HBM once and from that XCD's L2 after.
+// Workgroup = (16 state columns, batch.head), 4 waves; wave w owns state row tile w.  What
+// must follow one step after another is the S^T reads, DK/4 fp32 MFMAs (512 cycles at
+// DK = 64), the S^T write and one barrier.  M_n goes through LDS (double buffered, filled
+// from registers loaded kOpDepth chunks ahead) and is in operand registers a step ahead.
+// The products are formed transposed, S^T M^T, so that a lane's accumulator is four
+// consecutive columns of one state row: one 16-byte access each for Q_n and the record
+// where rows by lane took four.  The k-sum of each tile is split over four accumulators
+// (independent MFMA chains).  TRANS reads M_n transposed (the reverse scan takes A_n as
+// the forward scan does).  Workgroups go to the 8 XCDs round-robin by linear id: the
+// column groups of one batch.head are placed on one XCD, so each M_n comes from HBM once
+// and from that XCD's L2 after.
+// At 12 heads x 64 chunks, DK = 64, Dv = 128 (us, two scans / one): loads under branches,
+// each step waiting for all of them, 58.7 / 53.0; unconditional loads, products transposed
+// and M_n a step ahead 44.0 / 40.5.  Starting with the wave's own tile from registers
+// saves the wait for LDS but adds the largest products first (error 2.4e-7 against
+// 2.0e-7): not done.  Depth 6 and one workgroup per CU: equal here, 1.3x slower where
+// the launch holds several workgroups per CU; depth 2: 1.3x slower here.
 constexpr int kOpDepth = 4;
 constexpr int kXcds = 8;
+
+// four floats at any element address (dword alignment is all a 16-byte access needs)
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 
 template <int DK>
 struct OpPre {
   static constexpr int kMv = DK * DK / 4 / 256 > 0 ? DK * DK / 4 / 256 : 1;  // float4 of M per thread
-  static constexpr int kJt = (DK / 16 + 3) / 4;                             // row tiles per wave
   f32x4 m[kMv];
-  f32x4 q[kJt];
+  f32x4 q;
 };
 
 struct OpScanArgs {
@@ -301,7 +313,7 @@ __device__ __forceinline__ void opscan_body(const OpScanArgs &oa, int id, float 
   float *rec = oa.rec, *__restrict__ s_out = oa.s_out;
   int N = oa.N;
   const int Dv = oa.Dv, BH = oa.BH, rev = oa.rev;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane & 15, lq = lane >> 4;
   // linear id L on XCD L % 8: slot L / 8 of that XCD holds column group slot % ncg of
   // batch.head 8 (slot / ncg) + L % 8 (the grid is padded to whole groups per XCD)
@@ -320,105 +332,103 @@ __device__ __forceinline__ void opscan_body(const OpScanArgs &oa, int id, float 
   float *recb = rec + cell * qstride;
   auto order = [&](int i) { return rev ? N - 1 - i : i; };
 
-  // element (row, col) of a state-shaped [DK][Dv] matrix held by this lane for tile m, r
-  auto qoff = [&](int m, int r) { return static_cast<size_t>(16 * m + 4 * lq + r) * Dv + v0 + lr; };
-  auto load = [&](PR &pr, int n) {
+  // (waves past the row tiles repeat a tile's reads and write nothing)
+  const int mt = w % TT;
+  const bool mine = TT == 4 || w < TT;
+  // this lane's four elements of a state-shaped [DK][Dv] matrix: row 16 mt + lr, columns
+  // v0 + 4 lq + 0..3
+  const uint32_t qoff = static_cast<uint32_t>((16 * mt + lr) * Dv + v0 + 4 * lq);
+  // Every load and store of a step is unconditional (threads and waves without work repeat
+  // a valid address, steps past the end the last chunk), so the waits in the loop count
+  // exactly the later stages' loads: a load under a branch makes each step wait for all
+  // the loads in flight, its own included.
+  auto load = [&](PR &pr, int i) {
+    const int n = order(min(i, N - 1));
     const float *mp = Mb + static_cast<size_t>(n) * mstride;
 #pragma unroll
-    for (int e = 0; e < PR::kMv; ++e) {
-      const int idx = tid + 256 * e;  // float4 index
-      if (idx < DK * DK / 4) pr.m[e] = *reinterpret_cast<const f32x4 *>(mp + 4 * idx);
-    }
+    for (int e = 0; e < PR::kMv; ++e)
+      pr.m[e] = *reinterpret_cast<const f32x4 *>(mp + 4u * ((tid + 256 * e) % (DK * DK / 4)));
     const float *qp = Qb + static_cast<size_t>(n) * qstride;
-#pragma unroll
-    for (int j = 0; j < PR::kJt; ++j) {
-      const int m = w + 4 * j;
-      if (m < TT)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) pr.q[j][r] = qp[qoff(m, r)];
-    }
+    pr.q = *reinterpret_cast<const f32x4u *>(qp + qoff);
   };
   auto put_m = [&](const PR &pr, int buf) {
 #pragma unroll
     for (int e = 0; e < PR::kMv; ++e) {
-      const int idx = tid + 256 * e;
-      if (idx < DK * DK / 4) {
-        const int row = (4 * idx) / DK, col = (4 * idx) % DK;
-        *reinterpret_cast<f32x4 *>(&sM[buf][row * MS + col]) = pr.m[e];
+      const int idx = tid + 256 * e;  // float4 index
+      const int row = (4 * idx) / DK, col = (4 * idx) % DK;
+      if (DK * DK / 4 >= 256 || idx < DK * DK / 4) *reinterpret_cast<f32x4 *>(&sM[buf][row * MS + col]) = pr.m[e];
+    }
+  };
+  // M_n's operand rows of this wave's tile
+  auto read_m = [&](f32x4 (&av)[TT], int buf) {
+    const float *mrow = TRANS ? &sM[buf][4 * lq * MS + 16 * mt + lr] : &sM[buf][(16 * mt + lr) * MS + 4 * lq];
+#pragma unroll
+    for (int b = 0; b < TT; ++b) {
+      if (TRANS) {  // M^T[16 mt + lr][16 b + 4 lq + t] = M[16 b + 4 lq + t][16 mt + lr]
+#pragma unroll
+        for (int t = 0; t < 4; ++t) av[b][t] = mrow[(16 * b + t) * MS];
+      } else {
+        av[b] = *reinterpret_cast<const f32x4 *>(mrow + 16 * b);
       }
     }
   };
+  // S^T rows v0 + 4 lq + r of this lane's state row
+  auto put_s = [&](const f32x4 &x, int buf) {
+    if (mine)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) sS[buf][(4 * lq + r) * MS + 16 * mt + lr] = x[r];
+  };
 
-  f32x4 sreg[PR::kJt];
-#pragma unroll
-  for (int j = 0; j < PR::kJt; ++j) {
-    const int m = w + 4 * j;
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      sreg[j][r] = (s0 && m < TT) ? s0[static_cast<size_t>(bh) * qstride + qoff(m, r)] : 0.f;
-    if (m < TT) *reinterpret_cast<f32x4 *>(&sS[0][lr * MS + 16 * m + 4 * lq]) = sreg[j];
-  }
+  f32x4 sreg = {0.f, 0.f, 0.f, 0.f}, areg[TT];
+  if (s0) sreg = *reinterpret_cast<const f32x4u *>(s0 + static_cast<size_t>(bh) * qstride + qoff);
+  put_s(sreg, 0);
   PR pre[kOpDepth];
+  if (N > 0) {
 #pragma unroll
-  for (int d = 0; d < kOpDepth; ++d)
-    if (d < N) load(pre[d], order(d));
-  if (N > 0) put_m(pre[0], 0);
+    for (int d = 0; d < kOpDepth; ++d) load(pre[d], d);
+    put_m(pre[0], 0);
+    put_m(pre[1], 1);
+  }
+  __syncthreads();
+  read_m(areg, 0);
   __syncthreads();
 
-  // step i with the register stages of chunk i (cur) and of chunk i + 1 (nxt); the loop
+  // step i with the register stages of chunk i (cur) and of chunk i + 2 (nxt); the loop
   // below is unrolled by kOpDepth so the stage indices are compile-time constants
   auto step = [&](int i, PR &cur, const PR &nxt) {
-    const int n = order(i), buf = i & 1;
-    float *rp = recb + static_cast<size_t>(n) * qstride;
+    const int buf = i & 1;
+    f32x4 anext[TT], s4[TT];
 #pragma unroll
-    for (int j = 0; j < PR::kJt; ++j) {
-      const int m = w + 4 * j;
-      if (m < TT) {
+    for (int b = 0; b < TT; ++b) s4[b] = *reinterpret_cast<const f32x4 *>(&sS[buf][lr * MS + 16 * b + 4 * lq]);
+    __builtin_amdgcn_sched_barrier(0);
+    if (mine) *reinterpret_cast<f32x4u *>(recb + static_cast<size_t>(order(i)) * qstride + qoff) = sreg;
+    f32x4 acc[4] = {cur.q, {0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    read_m(anext, buf ^ 1);
+    put_m(nxt, buf);
+    load(cur, i + kOpDepth);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) rp[qoff(m, r)] = sreg[j][r];
-        f32x4 acc[4] = {cur.q[j], {0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-        const float *mrow = TRANS ? &sM[buf][4 * lq * MS + 16 * m + lr] : &sM[buf][(16 * m + lr) * MS + 4 * lq];
-        const float *srow = &sS[buf][lr * MS + 4 * lq];
+    for (int b = 0; b < TT; ++b)
 #pragma unroll
-        for (int b = 0; b < TT; ++b) {
-          f32x4 a4;
-          if (TRANS) {  // M^T[16 m + lr][16 b + 4 lq + t] = M[16 b + 4 lq + t][16 m + lr]
+      for (int t = 0; t < 4; ++t) acc[t] = mma4(s4[b][t], areg[b][t], acc[t]);
+    sreg = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+    put_s(sreg, buf ^ 1);
 #pragma unroll
-            for (int t = 0; t < 4; ++t) a4[t] = mrow[(16 * b + t) * MS];
-          } else {
-            a4 = *reinterpret_cast<const f32x4 *>(mrow + 16 * b);
-          }
-          const f32x4 s4 = *reinterpret_cast<const f32x4 *>(srow + 16 * b);
-#pragma unroll
-          for (int t = 0; t < 4; ++t) acc[t] = mma4(a4[t], s4[t], acc[t]);
-        }
-        sreg[j] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
-        *reinterpret_cast<f32x4 *>(&sS[buf ^ 1][lr * MS + 16 * m + 4 * lq]) = sreg[j];
-      }
-    }
-    if (i + 1 < N) put_m(nxt, buf ^ 1);
-    if (i + kOpDepth < N) load(cur, order(i + kOpDepth));
+    for (int j = 0; j < TT; ++j) areg[j] = anext[j];
     __syncthreads();
   };
   int i = 0;
   for (; i + kOpDepth <= N; i += kOpDepth) {
 #pragma unroll
-    for (int j = 0; j < kOpDepth; ++j) step(i + j, pre[j], pre[(j + 1) % kOpDepth]);
+    for (int j = 0; j < kOpDepth; ++j) step(i + j, pre[j], pre[(j + 2) % kOpDepth]);
   }
 #pragma unroll
   for (int j = 0; j < kOpDepth - 1; ++j)
-    if (i + j < N) step(i + j, pre[j], pre[(j + 1) % kOpDepth]);
-#pragma unroll
-  for (int j = 0; j < PR::kJt; ++j) {
-    const int m = w + 4 * j;
-    if (m < TT)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) s_out[static_cast<size_t>(bh) * qstride + qoff(m, r)] = sreg[j][r];
-  }
+    if (i + j < N) step(i + j, pre[j], pre[(j + 2) % kOpDepth]);
+  if (mine) *reinterpret_cast<f32x4u *>(s_out + static_cast<size_t>(bh) * qstride + qoff) = sreg;
 }
 
 template <int DK, bool TRANS, bool CELLS>
-__global__ void __launch_bounds__(256) gdn_opscan_f32_kernel(OpScanArgs oa) {
+__global__ void __launch_bounds__(256, 2) gdn_opscan_f32_kernel(OpScanArgs oa) {
   __shared__ __attribute__((aligned(16))) float sM[2][DK * opscan_ms<DK>()];
   __shared__ __attribute__((aligned(16))) float sS[2][kCols * opscan_ms<DK>()];
   opscan_body<DK, TRANS, CELLS>(oa, blockIdx.x, sM, sS);
@@ -428,7 +438,7 @@ __global__ void __launch_bounds__(256) gdn_opscan_f32_kernel(OpScanArgs oa) {
 // only A and G): workgroups [0, g1) walk the forward scan, the rest the reverse one (A
 // read transposed), so the two serial chains run side by side.
 template <int DK>
-__global__ void __launch_bounds__(256) gdn_opscan_pair_f32_kernel(OpScanArgs fwd, OpScanArgs rev, int g1) {
+__global__ void __launch_bounds__(256, 2) gdn_opscan_pair_f32_kernel(OpScanArgs fwd, OpScanArgs rev, int g1) {
   __shared__ __attribute__((aligned(16))) float sM[2][DK * opscan_ms<DK>()];
   __shared__ __attribute__((aligned(16))) float sS[2][kCols * opscan_ms<DK>()];
   const int id = blockIdx.x;

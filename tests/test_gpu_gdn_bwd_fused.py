@@ -103,3 +103,27 @@ def test_empty_sequence_passes_the_state_gradient(dtype):
     got = torch.autograd.grad([o, S], [*ts, s0], [do.to(DEV), dS.to(DEV)])
     assert all(a.shape == t.shape for a, t in zip(got, [*ts, s0]))
     assert torch.equal(got[-1].cpu(), dS)
+
+
+@pytest.mark.parametrize('transpose', [False, True])
+@pytest.mark.parametrize('dk,dv,shift', [(64, 128, 0), (64, 16, 1), (32, 48, 3), (16, 32, 0)])
+@pytest.mark.parametrize('N', [0, 1, 2, 3, 4, 5, 9])
+def test_operator_scan_depths(N, dk, dv, shift, transpose):
+    '''Chain lengths around the scan's load depth, operands and records at any element
+    address.  Bar: a step rounds dk products and sums of order one, 2^-24 (dk / 4 + 8), and
+    the contraction (|A| <= 1/2) keeps the sum over the steps below twice one step's.'''
+    from motif.ops.gdn_grad import opscan
+    g = torch.Generator().manual_seed(dk + N)
+
+    def rand(*shape):
+        n = torch.Size(shape).numel()
+        return torch.randn(n + shift, generator=g).to(DEV)[shift:].view(shape)
+    A = 0.5 * torch.linalg.qr(torch.randn(2, 3, max(N, 1), dk, dk, generator=g))[0][:, :, :N].to(DEV)
+    Q, S0 = rand(2, 3, N, dk, dv), rand(2, 3, dk, dv)
+    P, S = opscan(A, Q, S0, reverse=transpose, transpose=transpose)
+    ref = S0.double().cpu()
+    for n in (reversed(range(N)) if transpose else range(N)):
+        assert (P[:, :, n].double().cpu() - ref).abs().max() <= 2 ** -23 * (dk / 4 + 8) * ref.abs().max()
+        M = A[:, :, n].double().cpu()
+        ref = (M.transpose(-1, -2) if transpose else M) @ ref + Q[:, :, n].double().cpu()
+    assert (S.double().cpu() - ref).abs().max() <= 2 ** -23 * (dk / 4 + 8) * ref.abs().max()
