@@ -104,6 +104,7 @@ __device__ __forceinline__ uint4 ld16(const bf16_t *p) { return *reinterpret_cas
 // branch, and a tile costs two loads and its base.  The loads go to registers one tile ahead of the
 // stores.
 struct Stage2 { uint4 a, b; };
+constexpr uint32_t kPastEnd = 0x80000000u;  // past every tile's range
 struct StageSrc {
   const bf16_t *base;
   int64_t st;
@@ -115,6 +116,10 @@ struct StageSrc {
   __device__ __forceinline__ Stage2 load(int row0) const {
     const int rows = min(kT, nrows - row0);
     const buf_t buf = make_buf(base + int64_t(row0) * st, rows > 0 ? static_cast<uint32_t>(((rows - 1) * st + kBD) * 2) : 0u);
+    if (st < kBD) {  // rows that share elements (an expanded gradient): those past the end by number
+      const int r0 = 2 * (threadIdx.x & 15);
+      return {buf_ld16(buf, r0 < rows ? off : kPastEnd), buf_ld16(buf, r0 + 1 < rows ? off1 : kPastEnd)};
+    }
     return {buf_ld16(buf, off), buf_ld16(buf, off1)};
   }
 };
@@ -614,7 +619,9 @@ extern "C" int motif_chord_bwd(
   const uintptr_t al = reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v) |
                        reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(dout) |
                        reinterpret_cast<uintptr_t>(dq) | reinterpret_cast<uintptr_t>(dk) | reinterpret_cast<uintptr_t>(dv);
-  // (32-bit offsets inside a 32-row tile)
+  // (32-bit offsets inside a 32-row tile; the stride of a single row is never used)
+  if (L == 1) q_st = d_st = kBD;
+  if (S == 1) k_st = v_st = kBD;
   for (int64_t x : {q_st, k_st, v_st, d_st})
     if (x < 0 || x >= (int64_t(1) << 25)) return set_error(MOTIF_ERR_UNSUPPORTED, "chord_bwd: row stride out of range");
   if ((st & 7) != 0 || (al & 15) != 0) return set_error(MOTIF_ERR_UNSUPPORTED, "chord_bwd: need 16-byte aligned rows");

@@ -19,8 +19,8 @@
 // last kernel to read, ran its 24 64 x 64 x 64 products per chunk on one wave per SIMD (121 + 177
 // us), each operand read right before its use.  Here eight waves share a chunk (two per SIMD),
 // products are read a block ahead (gdn_tiles.h) and the last kernel needs only T, P and dS.
-// H = 12, T = 4096, dv = 128, bf16: operators 72 us, scans 60 us, gradients 144 us; forward and
-// backward through the op 509 -> 313 us.  Code a workgroup runs once is kept small (range-checked
+// H = 12, T = 4096, dv = 128, bf16: operators 71 us, scans 44 us, gradients 143 us; forward and
+// backward through the op 503 -> 298 us.  Code a workgroup runs once is kept small (range-checked
 // loads and stores instead of per-row selects, row vectors read four at a time): with a select per
 // element the last kernel's 93 KB of code outran the 64 KB instruction cache, 206 us.
 // Bound: the fp32 matrix rate (8.5 + 22 such products per chunk) and the barriers between them (one

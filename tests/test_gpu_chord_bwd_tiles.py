@@ -45,3 +45,35 @@ def test_broadcast_output_gradient():
     got = torch.autograd.grad(apply_chord_attention(*ts, log_n.to(DEV)), ts, one.to(DEV).expand(1, 4, 70, 64))
     for name, a, r in zip(('dq', 'dk', 'dv'), got[:3], ref[:3]):
         _close(a.cpu(), r, name)
+
+
+@pytest.mark.parametrize('L,S', [(1, 2), (33, 33), (70, 100)])
+def test_output_gradient_broadcast_over_rows(L, S):
+    '''One gradient row for every query (row stride 0, what a sum over the queries hands back):
+    the rows past L of the last tile share its elements and still count as zeros.'''
+    from motif.ops import apply_chord_attention
+    x = _inputs(2, 4, 2, L, S, 7 + L)
+    log_n = torch.log(torch.arange(S - L + 1, S + 1, dtype=torch.float32) + 1)[None].expand(2, L).contiguous()
+    row = x[7][:, :, :1]
+    _, ref = _grads_torch64(*x[:7], log_n, S - L, row.expand(2, 4, L, 64))
+    ts = [t.to(DEV).requires_grad_(True) for t in x[:7]]
+    dout = row.to(DEV).expand(2, 4, L, 64)
+    assert dout.stride(2) == 0 or L == 1
+    got = torch.autograd.grad(apply_chord_attention(*ts, log_n.to(DEV)), ts, dout)
+    for name, a, r in zip(('dq', 'dk', 'dv'), got[:3], ref[:3]):
+        _close(a.cpu(), r, f'{name} L={L}')
+
+
+def test_one_row_of_any_stride():
+    '''A single query and key row whose stride is past the staging offsets (never used).  One
+    key: dq and dk are zero up to the rounding of two 64-term dots of products below 16,
+    2 * 64 * 16 * 2^-24; dv is a bf16 rounding.'''
+    from motif.ops import apply_chord_attention
+    x = _inputs(1, 2, 1, 1, 1, 3)
+    log_n = torch.full((1, 1), 0.7)
+    _, ref = _grads_torch64(*x[:7], log_n, 0, x[7])
+    far = lambda t: t.to(DEV).as_strided(t.shape, (t.stride(0), t.stride(1), 1 << 26, 1))
+    ts = [far(t).requires_grad_(True) for t in x[:3]] + [t.to(DEV).requires_grad_(True) for t in x[3:7]]
+    got = torch.autograd.grad(apply_chord_attention(*ts, log_n.to(DEV)), ts, far(x[7]))
+    for name, a, r in zip(('dq', 'dk', 'dv'), got[:3], ref[:3]):
+        assert (a.double().cpu() - r).abs().max() <= 2 ** -8 * r.abs().max() + 2 ** -13, name
