@@ -1215,7 +1215,8 @@ static int launch_vector_dt(int dtype, const ChordArgs &a, int R, int D, const f
 }
 
 static bool head_dim_ok(int D) { return D == 16 || D == 32 || D == 64 || D == 128; }
-// bf16 at the model's head dim takes the MFMA kernels; everything else the vector kernel
+// bf16 at the model's head dim takes the kernels of this file; everything else chord_wide.hip's at
+// prefill and the vector kernel at decode
 static bool mfma_path(int dtype, int D) { return dtype == MOTIF_BF16 && D == kD; }
 
 // Workspace of the decode / fp32 paths: the bias table [H][S + 8] fp32 (read by the
