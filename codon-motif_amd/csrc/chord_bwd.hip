@@ -8,7 +8,8 @@
 //   d alpha_h = sum c dZ * (-(x^beta)),  d beta_h = sum c dZ * b ln x,
 //   d mu_h = sum c dZ * alpha beta x^(beta-1) sign(d - mu),  d ssmax_h = sum log_n dZ r
 // with x = |d - mu| + eps (the reference's backward: motif/ops/chord_attention.py:518-949,
-// :1348-1470).  P is rebuilt from the forward's log-sum-exp (log2 units), as there.
+// :1348-1470).  P is rebuilt from the forward's log-sum-exp (log2 units), as there.  s c dZ is
+// rounded to bf16 as one operand in both kernels.
 //
 // chord_bwd_dq_kernel: one workgroup per (head, 128 queries, chunk of key tiles, batch
 // row), a wave per 32 queries.  S^T = K Q^T and dP^T = V dO^T per 32-key tile on 32x32x16
@@ -30,9 +31,8 @@
 //
 // Bound by VALU issue (a tile's 1024 scores take ~10 instructions each and one exp2, its 12 or 16
 // MFMAs a third of that), so what is not per score is kept off the vector unit: tiles come through
-// range-checked buffers with fixed lane offsets, accumulators sit in ordinary registers, dQ's column
-// factor c s is taken after the sum, the dK / dV kernel reads a query's four values as one row that
-// the dQ kernel wrote.  B = 2, 12 heads, 2048 tokens: dQ 74 -> 57 us, dK / dV 73 -> 62, reductions
+// range-checked buffers with fixed lane offsets, accumulators sit in ordinary registers, the dK / dV
+// kernel reads a query's four values as one row that the dQ kernel wrote.  B = 2, 12 heads, 2048 tokens: dQ 74 -> 57 us, dK / dV 73 -> 62, reductions
 // 25 (three launches) -> 13 (one).
 #include <algorithm>
 #include <string>
@@ -246,12 +246,12 @@ __global__ void __launch_bounds__(256) chord_bwd_dq_kernel(ChordBwdArgs a) {
           const float rr = fmaf(s, sacc[r], wv.x);
           float p = fast_exp2(fmaf(cl, rr, -lse2));
           if constexpr (decltype(masked)::value) p = (qv && n0 + kk <= q_abs) ? p : 0.f;
-          const float g = p * (pacc[r] - delta);  // (dQ's factor c s is the column's: taken at the end)
+          const float g = p * (pacc[r] - delta);
           ss = fmaf(g, rr, ss);
           sa = fmaf(g, wv.y, sa);
           sb = fmaf(g, wv.z, sb);
           sm = fmaf(g, wv.w, sm);
-          dz[r] = g;
+          dz[r] = g * cs;  // (rounded to bf16 with its factor, as the dK / dV kernel rounds it)
         }
       };
       // every key of the tile at or before every query of the wave, all queries valid
@@ -270,11 +270,6 @@ __global__ void __launch_bounds__(256) chord_bwd_dq_kernel(ChordBwdArgs a) {
     __syncthreads();  // this tile's reads done, the next tile's stores visible
   }
 
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    dqacc[0][r] *= cs;
-    dqacc[1][r] *= cs;
-  }
   if (qv) {
     if (a.nsq == 1) {
       bf16_t *dst = a.dq + b * a.dq_sb + h * a.dq_sh + int64_t(my_q) * a.dq_st;

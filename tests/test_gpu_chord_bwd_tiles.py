@@ -1,6 +1,8 @@
 '''The Chord backward at the edges of its 32-row tiles, 6-tile chunks and 128-row blocks, with the
 output gradient in the [B, L, H, D] storage a layer hands back, inside a wider row and broadcast
 over heads; same reference and bars as tests/test_gpu_chord_bwd.py.'''
+import math
+
 import pytest
 import torch
 
@@ -77,3 +79,34 @@ def test_one_row_of_any_stride():
     got = torch.autograd.grad(apply_chord_attention(*ts, log_n.to(DEV)), ts, far(x[7]))
     for name, a, r in zip(('dq', 'dk', 'dv'), got[:3], ref[:3]):
         assert (a.double().cpu() - r).abs().max() <= 2 ** -8 * r.abs().max() + 2 ** -13, name
+
+
+@pytest.mark.parametrize('L', [70, 640])
+def test_dq_operand_rounding(L):
+    '''dQ is the bf16 of the fp32 sum of bf16(s c dZ) times K, one chunk of keys or several, with P
+    from the forward's own log-sum-exp (of its 16-bit P) and Delta from its 16-bit output.  P
+    carries a few 2^-20 from the exponential, so a share of 2^-20 / 2^-9 of the operands rounds
+    the other way (2^-8 each, of a sum of many: below 1e-4), and with that a share of 1e-4 / 2^-8
+    of the results (2^-8 each: 6e-4).  With the factor s c outside the rounding the distance is
+    that of two independent roundings, 3.4e-3.'''
+    from motif.ops import apply_chord_attention
+    from motif.ops.chord_attention import _launch
+    q, k, v, alpha, beta, mu, ssmax, dout = _inputs(1, 2, 2, L, L, 11 + L)
+    log_n = torch.log(torch.arange(1, L + 1, dtype=torch.float32))[None].contiguous()
+    ts = [t.to(DEV).requires_grad_(True) for t in (q, k, v, alpha, beta, mu, ssmax)]
+    out = apply_chord_attention(*ts, log_n.to(DEV))
+    dq = torch.autograd.grad(out, ts[0], dout.to(DEV))[0].double().cpu()
+    lse = torch.empty(1, 2, L, device=DEV)
+    with torch.no_grad():
+        _launch(*ts, log_n.to(DEV), 0, 0.125, 1e-5, torch.empty_like(out), lse)
+
+    col = lambda t: t.double().view(1, 2, 1, 1)  # noqa: E731
+    d = torch.arange(L)[None].double() - torch.arange(L)[:, None].double()
+    c = col(ssmax) * log_n.double().view(1, 1, L, 1)
+    bias = -col(alpha) * ((d - col(mu)).abs() + 1e-5) ** col(beta)
+    z = ((q.double() @ k.double().transpose(-1, -2)) * 0.125 + bias) * c
+    P = torch.exp2(z.masked_fill(d > 0, float('-inf')) * math.log2(math.e) - lse.double().cpu()[..., None])
+    delta = (dout.double() * out.detach().double().cpu()).sum(-1, keepdim=True)
+    dz = P * (dout.double() @ v.double().transpose(-1, -2) - delta)
+    want = ((dz * c * 0.125).bfloat16().double() @ k.double()).bfloat16().double()
+    assert ((dq - want).norm() / want.norm()).item() < 1e-3
