@@ -533,6 +533,14 @@ __global__ void __launch_bounds__(256) chord_bwd_reduce_kernel(ChordBwdArgs a, i
 // aimed at lie below 768 and 512), at least 6 tiles each and at most 8 chunks per block.  Swept at
 // 12 heads (whole backward, us; 1024 chunks of at least 16 tiles before): 2 x 2048 tokens 141 ->
 // 117, 4096 tokens (3 kv heads) 209 -> 186, 1024 tokens 57 -> 47, 700 tokens 57 -> 42.
+// A cut saves the tiles by which it shortens the longest block (1.25 us each on a CU of its own) and
+// costs each chunk's fp32 partial rows, written and read again: it is made where there are at most
+// `worth` chunks per tile saved.  Cut and whole measured side by side at 519 (dQ) and 399 (dK / dV)
+// sizes of 4 to 16 heads, 1 to 64 sequences and 64 to 4096 tokens: the rule takes the faster form or
+// one within 5% (dQ; worth 62), 7% (dK / dV, 42) and 8% (heads that share a kv head, whose partials
+// are written either way: 52).  Always cutting lost up to 31% where the launch filled the chip by
+// itself; 12 heads, us, cut / by the rule (and with the 1024-chunk plan): 16 x 512 tokens 104 / 87
+// (122), 8 x 512 75 / 60 (70), 16 x 256 59 / 42 (48).
 struct BwdPlan {
   int nqb, nkb, cq, nsq, ckv, nskv;
   bool kv_direct;
@@ -543,16 +551,22 @@ static BwdPlan plan_bwd(int B, int H, int Hkv, int L, int S, int q_start) {
   BwdPlan p{};
   p.nqb = (L + kBlk - 1) / kBlk;
   p.nkb = (S + kBlk - 1) / kBlk;
-  auto chunking = [](int64_t total, int maxt, int target, int &csize, int &ns) {
-    csize = static_cast<int>(std::max<int64_t>({6, (total + target - 1) / target, (maxt + 7) / 8}));
+  const int qt_end = (L + kT - 1) / kT;
+  auto chunking = [&](int nblocks, auto tiles, int target, int worth, int &csize, int &ns) {
+    int64_t total = 0, chunks = 0;
+    int maxt = 0;
+    for (int i = 0; i < nblocks; ++i) {
+      total += tiles(i);
+      maxt = std::max(maxt, tiles(i));
+    }
+    csize = static_cast<int>(std::max<int64_t>({6, (total * B * H + target - 1) / target, (maxt + 7) / 8}));
+    for (int i = 0; i < nblocks; ++i) chunks += (tiles(i) + csize - 1) / csize;
+    if (chunks * B * H > int64_t(worth) * (maxt - csize)) csize = std::max(csize, maxt);
     ns = std::max(1, (maxt + csize - 1) / csize);
   };
-  int64_t tq = 0, tkv = 0;
-  for (int qb = 0; qb < p.nqb; ++qb) tq += dq_tiles(qb, L, q_start);
-  const int qt_end = (L + kT - 1) / kT;
-  for (int kb = 0; kb < p.nkb; ++kb) tkv += std::max(0, qt_end - kv_first_tile(kb, q_start));
-  chunking(tq * B * H, p.nqb ? dq_tiles(p.nqb - 1, L, q_start) : 0, 640, p.cq, p.nsq);
-  chunking(tkv * B * H, qt_end, 384, p.ckv, p.nskv);
+  chunking(p.nqb, [&](int qb) { return dq_tiles(qb, L, q_start); }, 640, 62, p.cq, p.nsq);
+  chunking(p.nkb, [&](int kb) { return std::max(0, qt_end - kv_first_tile(kb, q_start)); }, 384, H == Hkv ? 42 : 52, p.ckv,
+           p.nskv);
   p.kv_direct = H == Hkv && p.nskv == 1;
   auto al = [](size_t x) { return (x + 255) / 256 * 256; };
   size_t off = al(static_cast<size_t>(B) * H * L * sizeof(float4));  // the query rows' values
