@@ -550,7 +550,7 @@ constexpr int kDecKeys = 4;                 // keys per lane group per step
 // its own running max / sum / output (merged at the end): the step has no cross-lane
 // traffic besides the LPK-lane dot-product sums.  This kernel serves the decode steps of
 // every dtype (fp32, bf16, fp16) and head dim (16, 32, 64, 128) -- bf16 at D = 64 has an MFMA
-// kernel -- and the prefills whose row strides chord_wide.hip does not take.
+// kernel -- and the prefills that chord_wide.hip does not take (row strides) or is slower at.
 template <typename T, int R, int D>
 __global__ void __launch_bounds__(256) chord_decode_kernel(ChordArgs a, const float *tab, int tab_n) {
   constexpr int LPK = D / 8, KG = 64 / LPK, kDecStep = KG * kDecKeys;
@@ -1219,6 +1219,31 @@ static bool head_dim_ok(int D) { return D == 16 || D == 32 || D == 64 || D == 12
 // prefill and the vector kernel at decode
 static bool mfma_path(int dtype, int D) { return dtype == MOTIF_BF16 && D == kD; }
 
+// Whether the fp32-arithmetic flash kernel (chord_wide.hip) beats the vector kernel on a prefill.
+// Both take time in rounds of workgroups, one per CU: the vector kernel's cover 8 rows of a kv
+// head's group, the flash kernel's 32 queries of one head, so from 8 queries on it has the fewer
+// and wins everywhere.  With fewer queries, many heads per kv head and large batches its tiles
+// are mostly padding and K / V are read once per head.  Fitted to 2218 sizes (1 to 32 heads per
+// kv head, 1 to 40 queries over 64 to 4096 keys, 1 to 128 sequences), in us: a round of the
+// vector kernel takes cv per 1000 keys, of the flash kernel cw and ow at its ends; the vector
+// kernel's second launch (its bias table) costs kTable.  At no size does the choice lose to the
+// vector kernel, whose call at fp32, 12 heads on 3, 3 tokens over 4096 takes 204 us at 64
+// sequences (flash: 275) and 103 at 8 (85); 16 heads on 1, 2 tokens over 4096 at 64: 109 (337).
+static bool wide_faster(const ChordArgs &a, int dtype, int D) {
+  const int group = a.H / a.Hkv;
+  const int64_t wv = int64_t(a.B) * a.Hkv * ((int64_t(group) * a.L + 7) / 8), ww = int64_t(a.B) * a.H * ((a.L + 31) / 32);
+  if (ww <= wv) return true;
+  struct Cost { float cv, cw, ow; };
+  static constexpr Cost k32[] = {{13.5f, 10.3f, .5f}, {23.f, 13.f, .5f}, {26.f, 22.5f, .5f}, {94.f, 57.f, 2.f}};
+  static constexpr Cost k16[] = {{12.f, 8.2f, 1.f}, {18.5f, 8.3f, 1.f}, {27.f, 13.f, 1.f}, {100.f, 24.f, 4.5f}};
+  constexpr float kTable = 4.f;
+  const Cost c = (dtype == MOTIF_F32 ? k32 : k16)[D == 16 ? 0 : D == 32 ? 1 : D == 64 ? 2 : 3];
+  const int cu = device_cu_count();
+  const float rv = static_cast<float>((wv + cu - 1) / cu), rw = static_cast<float>((ww + cu - 1) / cu);
+  const float keys = 1e-3f * static_cast<float>(std::min<int64_t>(a.S, int64_t(a.q_start) + a.L));
+  return rw * (c.cw * keys + c.ow) <= rv * c.cv * keys + kTable;
+}
+
 // Workspace of the decode / fp32 paths: the bias table [H][S + 8] fp32 (read by the
 // fp32 vector kernel; the bf16 MFMA kernel evaluates the bias in registers), then the
 // split partials [B][Hkv][splits][rows][D + 2] fp32.
@@ -1310,11 +1335,9 @@ extern "C" int motif_chord_fwd(
     const size_t need = tb + (a.splits > 1 ? static_cast<size_t>(B) * Hkv * a.splits * rows * (D + 2) * sizeof(float) : 0);
     if (!workspace || workspace_bytes < need)
       return set_error(MOTIF_ERR_INVALID, "chord_fwd: workspace too small (need " + std::to_string(need) + " bytes)");
-    // more rows than a decode step: the fp32-arithmetic flash kernel, unless its 32-bit tile
-    // offsets are too small for the row strides.  The vector kernel has no key split there and
-    // loses from its smallest call on: 12 heads, 3 kv heads, fp32, 3 tokens over 300: 27 against
-    // 30 us through the op; 3 over 4096: 85 against 102; 9 over 33 with 12 kv heads: 27 against 29.
-    if (!use_decode(H, Hkv, L, packed) && chord_wide_serves(a)) return launch_chord_wide(a, dtype, D, s);
+    // more rows than a decode step: the fp32-arithmetic flash kernel where its 32-bit tile offsets
+    // hold the row strides and it is the faster one
+    if (!use_decode(H, Hkv, L, packed) && chord_wide_serves(a) && wide_faster(a, dtype, D)) return launch_chord_wide(a, dtype, D, s);
     float *tab = static_cast<float *>(workspace);
     if (a.splits > 1) a.part = reinterpret_cast<float *>(static_cast<char *>(workspace) + tb);
     const int tn = table_len(S);

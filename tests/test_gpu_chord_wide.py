@@ -62,3 +62,12 @@ def test_wide_clipped_keys_and_strided_out():
     out = torch.empty(2, 50, 3, 64, device=DEV).transpose(1, 2)
     _check(*x, q_start=20, out=out)
     _check(*_inputs(1, 3, 3, 50, 400, 64, torch.float32, 8), q_start=100)
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float16])
+@pytest.mark.parametrize('B,H,Hkv,L,S,D', [(64, 16, 1, 2, 512, 64), (64, 8, 2, 3, 300, 64), (48, 16, 1, 1, 600, 32),
+                                           (64, 16, 1, 2, 40, 128)])
+def test_short_queries_in_large_batches(B, H, Hkv, L, S, D, dtype):
+    '''Sizes around the rule that leaves short query blocks of many heads per kv head to the
+    vector kernel.'''
+    _check(*_inputs(B, H, Hkv, L, S, D, dtype, S))
