@@ -1337,6 +1337,8 @@ extern "C" int motif_chord_fwd(
       return set_error(MOTIF_ERR_INVALID, "chord_fwd: workspace too small (need " + std::to_string(need) + " bytes)");
     // more rows than a decode step: the fp32-arithmetic flash kernel where its 32-bit tile offsets
     // hold the row strides and it is the faster one
+    if (L == 1) a.q_st = D;  // (the stride of a single row is not used)
+    if (S == 1) a.k_st = a.v_st = D;
     if (!use_decode(H, Hkv, L, packed) && chord_wide_serves(a) && wide_faster(a, dtype, D)) return launch_chord_wide(a, dtype, D, s);
     float *tab = static_cast<float *>(workspace);
     if (a.splits > 1) a.part = reinterpret_cast<float *>(static_cast<char *>(workspace) + tb);

@@ -71,3 +71,33 @@ def test_short_queries_in_large_batches(B, H, Hkv, L, S, D, dtype):
     '''Sizes around the rule that leaves short query blocks of many heads per kv head to the
     vector kernel.'''
     _check(*_inputs(B, H, Hkv, L, S, D, dtype, S))
+
+
+@pytest.mark.parametrize('stride', [(1 << 24) - 8, 1 << 24])
+def test_far_rows(stride):
+    '''Key rows on both sides of the stride that the flash kernel's 32-bit tile offsets hold (past
+    it: the vector kernel); 20 rows span 0.64 GB.'''
+    q, k, v, par = _inputs(1, 2, 1, 20, 20, 64, torch.float16, 4)
+    buf = torch.zeros(19 * stride + 64, dtype=torch.float16, device=DEV)
+    far = buf.as_strided((1, 1, 20, 64), (0, 0, stride, 1))
+    far.copy_(k)
+    ln = ochord.log_n_table(0, 20).float()[None].contiguous()
+    ref = ochord.chord_attention(q, k, v, *par, ln, 0, None)
+    got = ops.apply_chord_attention(q.to(DEV), far, v.to(DEV), *(p.to(DEV) for p in par), ln.to(DEV))
+    assert ((got.double().cpu() - ref).norm() / ref.norm()).item() < BAR[torch.float16]
+
+
+def test_far_single_rows():
+    '''The stride of a single row does not count: a query and a key row whose stride lies past the
+    tile offsets.'''
+    far = lambda t: t.to(DEV).as_strided(t.shape, (t.stride(0), t.stride(1), 1 << 26, 1))  # noqa: E731
+    q, k, v, par = _inputs(2, 16, 1, 1, 30, 64, torch.float32, 6)
+    ln = ochord.log_n_table(29, 1).float()[None].expand(2, 1).contiguous()
+    ref = ochord.chord_attention(q, k, v, *par, ln, 29, None)
+    got = ops.apply_chord_attention(far(q), k.to(DEV), v.to(DEV), *(p.to(DEV) for p in par), ln.to(DEV))
+    assert ((got.double().cpu() - ref).norm() / ref.norm()).item() < BAR[torch.float32]
+    q, k, v, par = _inputs(1, 2, 2, 9, 1, 64, torch.float32, 7)
+    ln = torch.full((1, 9), 0.5)
+    ref = ochord.chord_attention(q, k, v, *par, ln, 3, None)
+    got = ops.apply_chord_attention(q.to(DEV), far(k), far(v), *(p.to(DEV) for p in par), ln.to(DEV), q_start=3)
+    assert ((got.double().cpu() - ref).norm() / ref.norm()).item() < BAR[torch.float32]
