@@ -102,9 +102,12 @@ __device__ __forceinline__ uint4 ld16(const bf16_t *p) { return *reinterpret_cas
 // 32-row x 64 tile of [rows][64] bf16 rows, through a range-checked buffer that starts at the
 // tile's first row (uniform) and ends at row `nrows` of the matrix: rows past it read 0 with no
 // branch, and a tile costs two loads and its base.  The loads go to registers one tile ahead of the
-// stores.
+// stores.  ANY: rows that share elements (an expanded gradient), run backwards or lie past the
+// buffer's 32-bit offsets are told from those past the end by number, in kernels of their own (as
+// a branch here, its loads made every tile wait for all in flight: 10% of the whole backward).
 struct Stage2 { uint4 a, b; };
-constexpr uint32_t kPastEnd = 0x80000000u;  // past every tile's range
+constexpr int64_t kBufStride = int64_t(1) << 25;  // 31 rows and a bit stay below 2^31 bytes
+template <bool ANY>
 struct StageSrc {
   const bf16_t *base;
   int64_t st;
@@ -115,11 +118,13 @@ struct StageSrc {
         off1(off + static_cast<uint32_t>(2 * s)) {}
   __device__ __forceinline__ Stage2 load(int row0) const {
     const int rows = min(kT, nrows - row0);
-    const buf_t buf = make_buf(base + int64_t(row0) * st, rows > 0 ? static_cast<uint32_t>(((rows - 1) * st + kBD) * 2) : 0u);
-    if (st < kBD) {  // rows that share elements (an expanded gradient): those past the end by number
+    if constexpr (ANY) {
       const int r0 = 2 * (threadIdx.x & 15);
-      return {buf_ld16(buf, r0 < rows ? off : kPastEnd), buf_ld16(buf, r0 + 1 < rows ? off1 : kPastEnd)};
+      const bf16_t *p = base + (row0 + r0) * st + 8 * ((threadIdx.x & 127) >> 4);
+      const uint4 z = {0u, 0u, 0u, 0u};
+      return {r0 < rows ? ld16(p) : z, r0 + 1 < rows ? ld16(p + st) : z};
     }
+    const buf_t buf = make_buf(base + int64_t(row0) * st, rows > 0 ? static_cast<uint32_t>(((rows - 1) * st + kBD) * 2) : 0u);
     return {buf_ld16(buf, off), buf_ld16(buf, off1)};
   }
 };
@@ -142,6 +147,7 @@ __device__ __forceinline__ void stage_store(const Stage2 &g, int t, bf16_t *rows
 }
 
 // ------------------------------------------------------------------ dQ (+ Delta, parameter sums)
+template <bool ANY>
 __global__ void __launch_bounds__(256) chord_bwd_dq_kernel(ChordBwdArgs a) {
   const int h = blockIdx.x, qb = a.nqb - 1 - static_cast<int>(blockIdx.y);  // heaviest blocks first
   const int b = blockIdx.z / a.nsq, chunk = blockIdx.z - b * a.nsq;
@@ -158,7 +164,7 @@ __global__ void __launch_bounds__(256) chord_bwd_dq_kernel(ChordBwdArgs a) {
   const int kv_end = min(a.S, a.q_start + min(a.L, qb * kBlk + kBlk));
   // waves 0, 1 stage K (rows and K^T), 2, 3 V (rows); the first tile's loads go ahead of the rest
   const bool kside = w < 2;
-  const StageSrc src(kside ? a.k + b * a.k_sb + kvh * a.k_sh : a.v + b * a.v_sb + kvh * a.v_sh, kside ? a.k_st : a.v_st,
+  const StageSrc<ANY> src(kside ? a.k + b * a.k_sb + kvh * a.k_sh : a.v + b * a.v_sb + kvh * a.v_sh, kside ? a.k_st : a.v_st,
                      kv_end, tid & 127);
   Stage2 stg = src.load(t_begin * kT);
   const int qr = min(my_q, a.L - 1);
@@ -303,6 +309,7 @@ __global__ void __launch_bounds__(256) chord_bwd_dq_kernel(ChordBwdArgs a) {
 }
 
 // ------------------------------------------------------------------ dK, dV
+template <bool ANY>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) chord_bwd_dkdv_kernel(ChordBwdArgs a) {
   const int h = blockIdx.x, kb = blockIdx.y;
   const int b = blockIdx.z / a.nskv, chunk = blockIdx.z - b * a.nskv;
@@ -321,7 +328,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
   // tile's loads go ahead of the rest
   const bool qside = w < 2;
   const size_t rbase = (static_cast<size_t>(b) * a.H + h) * a.L;
-  const StageSrc src(qside ? a.q + b * a.q_sb + h * a.q_sh : a.dout + b * a.d_sb + h * a.d_sh, qside ? a.q_st : a.d_st, a.L,
+  const StageSrc<ANY> src(qside ? a.q + b * a.q_sb + h * a.q_sh : a.dout + b * a.d_sb + h * a.d_sh, qside ? a.q_st : a.d_st, a.L,
                      tid & 127);
   auto load_row = [&](int i0) {  // (queries past L: zeros, c = 0)
     const int n = min(kT, a.L - i0);
@@ -588,7 +595,7 @@ static BwdPlan plan_bwd(int B, int H, int Hkv, int L, int S, int q_start) {
 
 extern "C" size_t motif_chord_bwd_workspace_bytes(int B, int H, int Hkv, int L, int S, int q_start) {
   if (B <= 0 || H <= 0 || Hkv <= 0 || L < 0 || S < 0 || q_start < 0) return 0;
-  return motif::plan_bwd(B, H, Hkv, L, S, q_start).bytes;
+  return motif::plan_bwd(B, H, Hkv, L, S, q_start).bytes + 16;  // (up to 15 to align an odd base)
 }
 
 extern "C" int motif_chord_bwd(
@@ -628,15 +635,11 @@ extern "C" int motif_chord_bwd(
   const uintptr_t al = reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v) |
                        reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(dout) |
                        reinterpret_cast<uintptr_t>(dq) | reinterpret_cast<uintptr_t>(dk) | reinterpret_cast<uintptr_t>(dv);
-  // (32-bit offsets inside a 32-row tile; the stride of a single row is never used)
-  if (L == 1) q_st = d_st = kBD;
-  if (S == 1) k_st = v_st = kBD;
-  for (int64_t x : {q_st, k_st, v_st, d_st})
-    if (x < 0 || x >= (int64_t(1) << 25)) return set_error(MOTIF_ERR_UNSUPPORTED, "chord_bwd: row stride out of range");
   if ((st & 7) != 0 || (al & 15) != 0) return set_error(MOTIF_ERR_UNSUPPORTED, "chord_bwd: need 16-byte aligned rows");
   const BwdPlan pl = plan_bwd(B, H, Hkv, L, S, q_start);
-  if (!workspace || workspace_bytes < pl.bytes || (reinterpret_cast<uintptr_t>(workspace) & 15))
-    return set_error(MOTIF_ERR_INVALID, "chord_bwd: workspace too small or not 16-byte aligned (need " + std::to_string(pl.bytes) + " bytes)");
+  const size_t pad = -reinterpret_cast<uintptr_t>(workspace) & 15;  // (the size asked for holds it)
+  if (!workspace || workspace_bytes < pl.bytes + pad)
+    return set_error(MOTIF_ERR_INVALID, "chord_bwd: workspace too small (need " + std::to_string(pl.bytes + pad) + " bytes)");
   ChordBwdArgs a;
   a.q = static_cast<const bf16_t *>(q); a.q_sb = q_sb; a.q_sh = q_sh; a.q_st = q_st;
   a.k = static_cast<const bf16_t *>(k); a.k_sb = k_sb; a.k_sh = k_sh; a.k_st = k_st;
@@ -649,7 +652,7 @@ extern "C" int motif_chord_bwd(
   a.dk = static_cast<bf16_t *>(dk); a.dk_sb = dk_sb; a.dk_sh = dk_sh; a.dk_st = dk_st;
   a.dv = static_cast<bf16_t *>(dv); a.dv_sb = dv_sb; a.dv_sh = dv_sh; a.dv_st = dv_st;
   a.dparam = dparam;
-  char *ws = static_cast<char *>(workspace);
+  char *ws = static_cast<char *>(workspace) + pad;
   a.rows = reinterpret_cast<float4 *>(ws);
   a.pparam = reinterpret_cast<float *>(ws + pl.off_param);
   a.pq = reinterpret_cast<float *>(ws + pl.off_pq);
@@ -659,12 +662,15 @@ extern "C" int motif_chord_bwd(
   a.nqb = pl.nqb; a.nkb = pl.nkb;
   a.cq = pl.cq; a.nsq = pl.nsq; a.ckv = pl.ckv; a.nskv = pl.nskv; a.kv_direct = pl.kv_direct ? 1 : 0;
   a.scale = scale; a.eps = eps;
+  bool any = false;  // (a single row's stride is not used)
+  for (int64_t x : {q_st, d_st}) any |= L > 1 && (x < kBD || x >= kBufStride);
+  for (int64_t x : {k_st, v_st}) any |= S > 1 && (x < kBD || x >= kBufStride);
   int rc = MOTIF_OK;
   if (L > 0) {  // with no queries dK and dV are zero (the dK / dV pass below writes them)
-    chord_bwd_dq_kernel<<<dim3(H, pl.nqb, B * pl.nsq), dim3(256), 0, s>>>(a);
+    (any ? chord_bwd_dq_kernel<true> : chord_bwd_dq_kernel<false>)<<<dim3(H, pl.nqb, B * pl.nsq), dim3(256), 0, s>>>(a);
     if ((rc = check_launch("chord_bwd_dq_kernel"))) return rc;
   }
-  chord_bwd_dkdv_kernel<<<dim3(H, pl.nkb, B * pl.nskv), dim3(256), 0, s>>>(a);
+  (any ? chord_bwd_dkdv_kernel<true> : chord_bwd_dkdv_kernel<false>)<<<dim3(H, pl.nkb, B * pl.nskv), dim3(256), 0, s>>>(a);
   if ((rc = check_launch("chord_bwd_dkdv_kernel"))) return rc;
   auto blocks = [](int64_t rows) { return static_cast<int>((rows * (kBD / 4) + 255) / 256); };
   const int nkv = pl.kv_direct ? 0 : blocks(static_cast<int64_t>(B) * Hkv * S);

@@ -74,8 +74,8 @@ class ChordFunction(torch.autograd.Function):
         q, k, v, out, lse, alpha, beta, mu, ssmax, ln = ctx.saved_tensors
         B, H, L, D = q.shape
         Hkv, S = k.shape[1], k.shape[2]
-        # (the kernels read dout's own rows, expanded ones too; strides past their offsets are copied)
-        dout = _aligned(dout if dout.stride(-1) == 1 and dout.stride(2) < 1 << 25 else dout.contiguous())
+        # (the kernels read dout's own rows, expanded ones too)
+        dout = _aligned(dout if dout.stride(-1) == 1 else dout.contiguous())
         dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
         lib = _lib.lib()
         d_params = torch.empty((4, H), dtype=torch.float32, device=q.device)

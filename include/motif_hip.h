@@ -353,8 +353,7 @@ int motif_chord_fwd(
  *   workspace: motif_chord_bwd_workspace_bytes(B, H, Hkv, L, S, q_start) bytes (row sums
  *   dout . out and the fp32 partials of the chunked causal loops).  Needs 0 <= q_start
  *   and q_start + L <= S.  Results do not depend on the run: partials are summed in a
- *   fixed order.  Rows start on 16-byte boundaries, the workspace too; row strides of q, k,
- *   v and dout lie in [0, 2^25) elements (that of a single row is not used).
+ *   fixed order.  Rows start on 16-byte boundaries; any row strides, any workspace address.
  */
 size_t motif_chord_bwd_workspace_bytes(int B, int H, int Hkv, int L, int S, int q_start);
 int motif_chord_bwd(

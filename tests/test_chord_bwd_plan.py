@@ -8,7 +8,7 @@ from motif.ops import _lib
 def _planes(B, H, Hkv, L, S):
     '''(dQ, dK / dV) partial planes, and the bytes that every plan needs.'''
     q_start = S - L
-    got = _lib.lib().motif_chord_bwd_workspace_bytes(B, H, Hkv, L, S, q_start)
+    got = _lib.lib().motif_chord_bwd_workspace_bytes(B, H, Hkv, L, S, q_start) - 16  # (room to align an odd base)
     al = lambda n: -(-n // 256) * 256  # noqa: E731
     nqb = -(-L // 128)
     hits = []

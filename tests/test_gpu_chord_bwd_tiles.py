@@ -110,3 +110,43 @@ def test_dq_operand_rounding(L):
     dz = P * (dout.double() @ v.double().transpose(-1, -2) - delta)
     want = ((dz * c * 0.125).bfloat16().double() @ k.double()).bfloat16().double()
     assert ((dq - want).norm() / want.norm()).item() < 1e-3
+
+
+@pytest.mark.parametrize('form', ['far', 'backwards', 'workspace'])
+def test_entry_takes_any_row_stride_and_workspace(form):
+    '''motif_chord_bwd itself on rows 2^25 elements apart (0.3 GB each), rows that run backwards,
+    and a workspace off 16-byte boundaries: the bits of the plain call.'''
+    from motif.ops import _lib
+    from motif.ops.chord_attention import _launch
+    q, k, v, alpha, beta, mu, ssmax, dout = (t.to(DEV) for t in _inputs(1, 1, 1, 5, 5, 9))
+    log_n = torch.log(torch.arange(1, 6, dtype=torch.float32, device=DEV))[None].contiguous()
+    out, lse = torch.empty_like(q), torch.empty(1, 1, 5, device=DEV)
+    with torch.no_grad():
+        _launch(q, k, v, alpha, beta, mu, ssmax, log_n, 0, 0.125, 1e-5, out, lse)
+
+    def arg(t):
+        if form == 'far':
+            buf = torch.zeros((4 << 25) + 64, dtype=t.dtype, device=DEV)
+            rows = buf.as_strided(t.shape, (0, 0, 1 << 25, 1))
+            rows.copy_(t)
+            return buf, [buf.data_ptr(), 0, 0, 1 << 25]
+        if form == 'backwards':
+            buf = t.flip(2).contiguous()
+            return buf, [buf[0, 0, 4].data_ptr(), 0, 0, -64]
+        return t, _lib.t4(t)
+
+    def call(args, shift):
+        grads = [torch.empty_like(t) for t in (q, k, v)]
+        par = torch.empty(4, 1, device=DEV)
+        n = int(_lib.lib().motif_chord_bwd_workspace_bytes(1, 1, 1, 5, 5, 0))
+        ws = torch.empty(n + 16, dtype=torch.uint8, device=DEV)
+        a = [x for _, t in args[:3] for x in t] + _lib.t4(out) + args[3][1]
+        rc = _lib.lib().motif_chord_bwd(
+            *a, lse.data_ptr(), *(t.data_ptr() for t in (alpha, beta, mu, ssmax, log_n)), 5, 1,
+            *(x for t in grads for x in _lib.t4(t)), par.data_ptr(), 1, 1, 1, 5, 5, 64, 0, 0.125, 1e-5,
+            ws.data_ptr() + shift, n, _lib.chord_dtype_code(q.dtype), _lib.stream_ptr(q.device))
+        _lib.check(rc, 'motif_chord_bwd')
+        return [*grads, par]
+    plain = call([(t, _lib.t4(t)) for t in (q, k, v, dout)], 0)
+    got = call([arg(t) for t in (q, k, v, dout)], 4 if form == 'workspace' else 0)
+    assert all(torch.equal(a, b) for a, b in zip(got, plain))
