@@ -139,10 +139,11 @@ def _check_params(alpha, beta, mu, ssmax, num_heads):
 
 
 def _aligned(t):
-    '''Rows must start on 16-byte boundaries for the vector loads.'''
+    '''Rows must start on 16-byte boundaries for the vector loads.  (A copy where they do not:
+    contiguous() returns a contiguous tensor as it is, whatever its address.)'''
     per16 = 16 // t.element_size()
     ok = t.data_ptr() % 16 == 0 and all(s % per16 == 0 for s in t.stride()[:-1])
-    return t if ok else t.contiguous()
+    return t if ok else torch.empty(t.shape, dtype=t.dtype, device=t.device).copy_(t)
 
 
 def _check_out(out, shape, dtype, device):
