@@ -67,7 +67,7 @@ def linear_rows(x, weight, epilogue='none', aux=None, aux2=None, out=None, out2=
     code = EPILOGUES[epilogue]
     if wants_grad(x, weight, aux, aux2):
         return _torch_form(x, weight, code, aux, aux2)
-    if code == 0 and out is None and x.is_contiguous():  # (no views to build)
+    if code == 0 and aux is None and aux2 is None and out is None and x.is_contiguous():  # (no views to build)
         K, N = x.shape[-1], weight.shape[0]
         y = torch.empty(*x.shape[:-1], N, dtype=x.dtype, device=x.device)
         rc = _lib.lib().motif_linear_rows(x.data_ptr(), K, weight.data_ptr(), weight.stride(0), y.data_ptr(), N,
