@@ -419,10 +419,10 @@ extern "C" int motif_gdn_recurrent_fwd(
 extern "C" size_t motif_gdn_chunk_workspace_bytes(int H, int dk, int dv, int chunk, int total_chunks) {
   if (H <= 0 || dk <= 0 || dv <= 0 || chunk <= 0 || total_chunks <= 0) return 0;
   // whichever of the bf16 MFMA, fp32 MFMA and vector kernels serves the inputs
-  size_t mfma = chunk_mfma_supported(dk, dv, chunk) ? chunk_mfma_workspace_bytes(H, dk, dv, total_chunks) : 0;
-  // (the fp32 MFMA kernels' dk dk + dk dv + 64 dk floats are within the vector kernels' share)
+  const size_t mfma = chunk_mfma_supported(dk, dv, chunk) ? chunk_mfma_workspace_bytes(H, dk, dv, total_chunks) : 0;
+  const size_t f32 = chunk_f32_supported(dk, dv, chunk) ? chunk_f32_workspace_bytes(H, dk, dv, total_chunks) : 0;
   const size_t per = static_cast<size_t>(chunk) * (1 + dk + dv + chunk);
-  return std::max(mfma, per * H * total_chunks * sizeof(float));
+  return std::max({mfma, f32, per * H * total_chunks * sizeof(float)});
 }
 
 static int chunk_fwd_impl(
