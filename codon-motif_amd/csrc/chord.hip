@@ -1215,8 +1215,8 @@ static int launch_vector_dt(int dtype, const ChordArgs &a, int R, int D, const f
 }
 
 static bool head_dim_ok(int D) { return D == 16 || D == 32 || D == 64 || D == 128; }
-// bf16 at the model's head dim takes the kernels of this file; everything else chord_wide.hip's at
-// prefill and the vector kernel at decode
+// bf16 at the model's head dim takes the MFMA kernels of this file; everything else the vector kernel
+// at decode, and at prefill chord_wide.hip's or the vector kernel (wide_faster)
 static bool mfma_path(int dtype, int D) { return dtype == MOTIF_BF16 && D == kD; }
 
 // Whether the fp32-arithmetic flash kernel (chord_wide.hip) beats the vector kernel on a prefill.

@@ -32,8 +32,10 @@
 // Bound by VALU issue (a tile's 1024 scores take ~10 instructions each and one exp2, its 12 or 16
 // MFMAs a third of that), so what is not per score is kept off the vector unit: tiles come through
 // range-checked buffers with fixed lane offsets, accumulators sit in ordinary registers, the dK / dV
-// kernel reads a query's four values as one row that the dQ kernel wrote.  B = 2, 12 heads, 2048 tokens: dQ 74 -> 57 us, dK / dV 73 -> 62, reductions
-// 25 (three launches) -> 13 (one).
+// kernel reads a query's four values as one row that the dQ kernel wrote.  B = 2, 12 heads, 2048
+// tokens: dQ 73 -> 57 us, dK / dV 72 -> 62, reductions 26 (three launches) -> 14 (one).  Whole
+// backward, back to back: that size 165 -> 131 us, 4096 tokens (3 kv heads) 282 -> 193, 1024 tokens
+// 71 -> 45, 16 x 512 tokens 125 -> 88.
 #include <algorithm>
 #include <string>
 
@@ -538,8 +540,9 @@ __global__ void __launch_bounds__(256) chord_bwd_reduce_kernel(ChordBwdArgs a, i
 // Chunk sizes: about as many full chunks over the whole causal loop as the kernel's workgroups fit
 // on the chip at once (dQ: three per CU, dK / dV: two; blocks end in shorter chunks, so the counts
 // aimed at lie below 768 and 512), at least 6 tiles each and at most 8 chunks per block.  Swept at
-// 12 heads (whole backward, us; 1024 chunks of at least 16 tiles before): 2 x 2048 tokens 141 ->
-// 117, 4096 tokens (3 kv heads) 209 -> 186, 1024 tokens 57 -> 47, 700 tokens 57 -> 42.
+// 12 heads (the two kernels and the reductions in a loop, us; 1024 chunks of at least 16 tiles against
+// these): 2 x 2048 tokens 141 -> 117, 4096 tokens (3 kv heads) 209 -> 186, 1024 tokens 57 -> 47, 700
+// tokens 57 -> 42.
 // A cut saves the tiles by which it shortens the longest block (1.25 us each on a CU of its own) and
 // costs each chunk's fp32 partial rows, written and read again: it is made where there are at most
 // `worth` chunks per tile saved.  Cut and whole measured side by side at 519 (dQ) and 399 (dK / dV)

@@ -6,21 +6,26 @@
 // ceil(S / 32 / NW) tiles and short prompts still fill the chip.  The waves share no keys, so
 // nothing is staged: K and V come from global memory (L2) straight into the operand registers.
 //   S^T = K Q^T    lane l: key l % 32 of the tile against query l % 32.  fp32 inputs take
-//                  v_mfma_f32_32x32x2_f32 in two chains (the lane half h holds features
-//                  8 j + 4 h + 0..3, so both operands are 16-byte pieces of a row); 16-bit
-//                  inputs take 32x32x16, whose products are exact and whose sums are fp32.
+//                  v_mfma_f32_32x32x2_f32 in D / 8 chains of eight features, two side by
+//                  side, summed pairwise (the lane half h holds features 8 j + 4 h + 0..3, so
+//                  both operands are 16-byte pieces of a row); 16-bit inputs take 32x32x16,
+//                  whose products are exact and whose sums are fp32.
 //   O^T += V^T P^T on v_mfma_f32_32x32x2_f32 for every type: P stays fp32, straight from the
 //                  score accumulators (register r of half h is key 8 (r / 4) + 4 h + r % 4), V
 //                  converts to fp32 exactly.  Row m of output tile t is feature VD m + t
 //                  (VD = D / 32), so a lane's V piece of a key is VD consecutive features.
-// The next tile's K is requested when S^T is done and this tile's V before it, so each load has
-// a product (64 D / 32 x 64 cycles) to arrive in.  The distance bias of a tile depends on 63
-// distances: each lane evaluates one into a wave-private LDS window.
-// Bound: the fp32 matrix rate (64 flop a cycle and SIMD): 64 MFMAs of 64 cycles per 32 x 32
-// scores at D = 64 fp32, half of that for 16-bit inputs.  Measured against the vector kernel
-// that served these shapes (12 heads, 3 kv heads): fp32 1023 tokens 34 us (was 143), 4096 tokens
-// 324 us (1376), 3 tokens over 4096 85 us (102); fp16 1023 tokens 22 us (147); bf16 D = 128 1000
-// tokens 37 us (380).  Error against 64 bits, fp32: 3.7e-7 (3.9e-7).
+// This tile's V is requested before S^T, the next tile's K when S^T is done.  K has the softmax and
+// the whole O product to arrive in (D / 2 MFMAs of 64 cycles: 2048 cycles at D = 64).  V has the
+// score product and the softmax: D / 2 MFMAs of 64 cycles for fp32, but only D / 16 of 32 cycles
+// (128 at D = 64) for 16-bit inputs.  The distance bias of a tile depends on 63 distances: each
+// lane evaluates one into a wave-private LDS window.
+// Bound: per 32 x 32 scores at D = 64, 64 fp32 MFMAs of 64 cycles (32 and four of 32 cycles for
+// 16-bit inputs), where the query blocks fill the chip: the matrix pipe is busy 58% of the time at
+// 4096 tokens, fp32.  At 1023 tokens (28%; fp16 21%) the 384 workgroups, one per CU, are a round
+// and a half, and the longest rows' chain of tiles sets its length.  Kernel time under the tracer, 12 heads, 3 kv heads, in
+// us (and of the vector kernel that served these shapes, with its bias table's launch): fp32 1023
+// tokens 34.5 (151), 4096 tokens 325 (1355), 3 tokens over 4096 82 (101); fp16 1023 tokens 22 (148);
+// bf16 D = 128 1000 tokens 36 (381).  Error against 64 bits, fp32: 3.7e-7 (4.1e-7).
 #include <algorithm>
 
 #include "capi_internal.h"

@@ -307,8 +307,9 @@ __device__ __forceinline__ void opscan_body(const OpScanArgs &oa, int id, float 
                                             float (*sS)[kCols * opscan_ms<DK>()]) {
   constexpr int TT = DK / 16, MS = opscan_ms<DK>();  // row tiles; LDS row stride
   using PR = OpPre<DK>;
-  // (CELLS: rec may be Q -- each lane reads an element of Q_n kOpDepth chunks before it
-  // overwrites that element with S_n -- so neither is restrict)
+  // (rec may be Q, in the CELLS form and in the pair that the whole backward runs: each lane
+  // reads an element of Q_n kOpDepth chunks before it overwrites that element with S_n -- so
+  // neither is restrict)
   const float *__restrict__ M = oa.M, *Q = oa.Q, *__restrict__ s0 = oa.s0;
   float *rec = oa.rec, *__restrict__ s_out = oa.s_out;
   int N = oa.N;

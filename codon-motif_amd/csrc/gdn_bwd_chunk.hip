@@ -1,6 +1,9 @@
 // GatedDeltaNet chunk backward, the per-chunk parts as entry points of their own (gfx950, fp32 on
 // v_mfma_f32_32x32x2_f32): motif_gdn_bwd_prep_f32 and motif_gdn_bwd_chunk_f32.  The op's backward
-// runs motif_gdn_chunk_bwd (gdn_bwd_fused.hip).
+// runs motif_gdn_chunk_bwd (gdn_bwd_fused.hip) and reaches none of this: the two stay as C entry
+// points (with wrappers in ops/gdn_grad.py) for callers that hold chunked fp32 tensors or need a
+// piece by itself -- W, U, T and dX, or the gradients around scans of their own -- which the one
+// call does not give.
 //
 // The reference differentiates its chunked rule in three pieces (motif/ops/gated_deltanet.py):
 // the chunk preparation (`_PrepareChunksFunction.backward`, :180-260, the triangular solve

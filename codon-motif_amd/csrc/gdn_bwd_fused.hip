@@ -1,5 +1,7 @@
 // GatedDeltaNet chunk backward (gfx950): the whole backward of the chunked rule from the caller's
-// own tensors (fp32 or bf16, any strides) to their gradients, fp32 inside, in three launches:
+// own tensors (fp32 or bf16; unit feature strides, rows of q, k, v and dout apart and on
+// four-element boundaries, row strides below 2^23; any batch and head strides on such boundaries)
+// to their gradients, fp32 inside, in three launches:
 //   gdn_bwd_operators   one workgroup per (chunk, batch * head): T = (I - A)^{-1} and the two scans'
 //                       per-chunk operators
 //                         A_n = e^{gamma_C} I - M1 K',  H_n = M1 V',  G_n = Q'^T dO,
@@ -20,11 +22,12 @@
 // us), each operand read right before its use.  Here eight waves share a chunk (two per SIMD),
 // products are read a block ahead (gdn_tiles.h) and the last kernel needs only T, P and dS.
 // H = 12, T = 4096, dv = 128, bf16: operators 71 us, scans 44 us, gradients 143 us; forward and
-// backward through the op 503 -> 298 us.  Code a workgroup runs once is kept small (range-checked
+// backward through the op 509 -> 298 us.  Code a workgroup runs once is kept small (range-checked
 // loads and stores instead of per-row selects, row vectors read four at a time): with a select per
 // element the last kernel's 93 KB of code outran the 64 KB instruction cache, 206 us.
-// Bound: the fp32 matrix rate (8.5 + 22 such products per chunk) and the barriers between them (one
-// workgroup per CU: 120-155 KB of LDS).
+// Bound: the phases' chains.  The 8.5 + 22 such products per chunk keep the matrix pipe busy 31% (operators)
+// and 41% (gradients) of the time; with one workgroup per CU (120-155 KB of LDS) nothing else runs
+// while its waves wait at a barrier or for a phase's LDS round trips.
 #include <type_traits>
 
 #include "gdn_internal.h"

@@ -13,10 +13,11 @@
 // The form this replaced (row-by-row substitution of [W | U] and a scan holding three
 // products per chunk, on the vector unit) put every chunk's products into the serial chain:
 // 17 us a chunk.  Here only one dk x dk x dv product per chunk is serial.  Measured (prep +
-// scan + output): 30 us at B = 1, H = 4, T = 256, dk = dv = 64 (19.5 + 5.2 + 5.7; was 110), 144 us
-// at H = 12, T = 4096, dv = 128 (78 + 41 + 20; was 1220).  The prep is bound by its MFMA chains
-// and the LDS round trips between its phases (one workgroup per CU), the scan by the chain.
-// Its error against 64 bits is the smaller one too (2.4e-7 against 2.8e-7 relative).
+// scan + output): 30 us at B = 1, H = 4, T = 256, dk = dv = 64 (19.4 + 5.2 + 5.7; was 110), 138 us
+// at H = 12, T = 4096, dv = 128 (77 + 41 + 20; was 1220).  The prep is bound by its MFMA chains (32
+// terms each) and the LDS round trips between its phases (one workgroup per CU; the matrix pipe is
+// busy 27% of the time), the scan by the chain.  Its error against 64 bits is the smaller one too
+// (4.0e-7 against 4.5e-7 relative at T = 256).
 #include <algorithm>
 #include <type_traits>
 

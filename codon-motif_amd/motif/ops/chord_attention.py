@@ -3,10 +3,11 @@
 `apply_chord_attention` keeps the reference signature, defaults, validation
 messages and exception types (motif/ops/chord_attention.py:1557-1625 with
 `_check_tensors` :966-1011 and `_check_params` :1448-1472).  The launcher
-picks the bf16 MFMA flash kernel for prefill shapes (head dim 64; other head dims,
-fp16 and fp32 the fp32-arithmetic flash kernel) and the split-K decode kernels when
-a kv head serves at most 8 query rows (GQA group x L), which is the reference's
-long-KV / short-Q split path (:1128-1229).  fp32 inputs are multiplied and summed in
+picks the bf16 MFMA flash kernel for prefill shapes (head dim 64; for other head dims,
+fp16 and fp32 the fp32-arithmetic flash kernel, or the vector kernel where that is the
+faster one: few queries in large batches) and the split-K decode kernels when a kv head
+serves at most 8 query rows (GQA group x L), which is the reference's long-KV / short-Q
+split path (:1128-1229).  fp32 inputs are multiplied and summed in
 fp32 on every path (the accuracy mode).
 `apply_chord_attention_varlen` adds packed sequences (new) and
 `chord_decode_cursor` the decode step over a fixed-capacity cache whose length
