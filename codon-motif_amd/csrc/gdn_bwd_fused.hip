@@ -28,6 +28,7 @@
 // Bound: the phases' chains.  The 8.5 + 22 such products per chunk keep the matrix pipe busy 31% (operators)
 // and 41% (gradients) of the time; with one workgroup per CU (120-155 KB of LDS) nothing else runs
 // while its waves wait at a barrier or for a phase's LDS round trips.
+#include <algorithm>
 #include <type_traits>
 
 #include "gdn_internal.h"
@@ -39,6 +40,7 @@ namespace {
 
 constexpr int kC = 64, kDK = 64, kLD = 65, kThreads = 512;
 constexpr int kPlane = kC * kLD;
+constexpr int kMaxGrid = 65535;  // second and third grid dimensions
 
 struct View {  // [B, H, L, (features)] tensor
   const void *p;
@@ -50,6 +52,7 @@ struct BwdArgs {
   View dq, dk, dv, dbeta, dg;  // (written)
   float *T, *A, *P, *dS;       // [BH * N][64][64], [..][dk][dk], [..][dk][dv] (H_n, then P_n), [..][dk][dv] (G_n, then dS_n)
   int H, L, N;
+  int b0;                      // first batch row of the launch
 };
 
 template <typename T>
@@ -101,7 +104,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
   float *sK = sm + LD::k, *sQ = sm + LD::q, *sV = sm + LD::v, *sDo = sm + LD::d, *sN = sm + LD::n, *sT = sm + LD::t,
         *sAt = sm + LD::at;
   float *sGam = sm + LD::gam, *sE = sm + LD::eg, *sKd = sm + LD::kd, *sB = sm + LD::be, *xs = sm + LD::xs;
-  const int n = blockIdx.x, hd = blockIdx.y, b = blockIdx.z, t0 = n * kC, len = min(kC, a.L - t0);
+  const int n = blockIdx.x, hd = blockIdx.y, b = a.b0 + blockIdx.z, t0 = n * kC, len = min(kC, a.L - t0);
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int i = lane & 31, h = lane >> 5;
   const size_t cell = (static_cast<size_t>(b) * a.H + hd) * a.N + n;
@@ -264,7 +267,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
   float *sK = sm + LD::k, *sT = sm + LD::t, *sAt = sm + LD::at, *b0 = sm + LD::b0, *b1 = sm + LD::b1, *b2 = sm + LD::b2,
         *b3 = sm + LD::b3, *b4 = sm + LD::b4;
   float *sGam = sm + LD::gam, *sE = sm + LD::eg, *sDec = sm + LD::dec, *sB = sm + LD::be;
-  const int n = blockIdx.x, hd = blockIdx.y, b = blockIdx.z, t0 = n * kC, len = min(kC, a.L - t0);
+  const int n = blockIdx.x, hd = blockIdx.y, b = a.b0 + blockIdx.z, t0 = n * kC, len = min(kC, a.L - t0);
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int i = lane & 31, h = lane >> 5;
   // each wave owns the 32 x 32 tile (r0, c0) of every 64 x 64 result of its group (waves 0-3, 4-7)
@@ -572,17 +575,24 @@ size_t ws_floats(int64_t BH, int N, int dv) {
 }
 
 template <typename T, int DV>
-int launch_bwd(const BwdArgs &a, int B, const float *S0, const float *dS_final, float *dS0, float *s_scratch, hipStream_t s) {
-  const dim3 grid(a.N, a.H, B), block(kThreads);
+int launch_bwd(BwdArgs a, int B, const float *S0, const float *dS_final, float *dS0, float *s_scratch, hipStream_t s) {
+  const dim3 block(kThreads);
+  // (a launch takes 65535 batch rows)
+  auto grid = [&] { return dim3(a.N, a.H, std::min(B - a.b0, kMaxGrid)); };
   constexpr size_t smem1 = OpLds<DV>::floats * 4, smem2 = GradLds::floats * 4;
   if (int rc = set_smem(gdn_bwd_operators<T, DV>, smem1, "gdn_bwd_operators")) return rc;
-  gdn_bwd_operators<T, DV><<<grid, block, smem1, s>>>(a);
-  if (int rc = check_launch("gdn_bwd_operators")) return rc;
+  for (a.b0 = 0; a.b0 < B; a.b0 += kMaxGrid) {
+    gdn_bwd_operators<T, DV><<<grid(), block, smem1, s>>>(a);
+    if (int rc = check_launch("gdn_bwd_operators")) return rc;
+  }
   if (int rc = motif_gdn_opscan_pair_f32(a.A, a.P, S0, a.P, s_scratch, a.dS, dS_final, a.dS, dS0, B * a.H, a.N, kDK, DV, s))
     return rc;
   if (int rc = set_smem(gdn_bwd_grads<T, DV>, smem2, "gdn_bwd_grads")) return rc;
-  gdn_bwd_grads<T, DV><<<grid, block, smem2, s>>>(a);
-  return check_launch("gdn_bwd_grads");
+  for (a.b0 = 0; a.b0 < B; a.b0 += kMaxGrid) {
+    gdn_bwd_grads<T, DV><<<grid(), block, smem2, s>>>(a);
+    if (int rc = check_launch("gdn_bwd_grads")) return rc;
+  }
+  return MOTIF_OK;
 }
 
 }  // namespace
@@ -617,7 +627,7 @@ extern "C" int motif_gdn_chunk_bwd(
   if (!q || !k || !v || !beta || !g || !dout || !dq || !dk_ || !dv_ || !dbeta || !dg || !dstate_in)
     return set_error(MOTIF_ERR_INVALID, "gdn_chunk_bwd: NULL pointer");
   const int N = (L + kC - 1) / kC;
-  if (H > 65535 || B > 65535 || int64_t(B) * H * N >= (int64_t(1) << 31))
+  if (H > kMaxGrid || int64_t(B) * H * N >= (int64_t(1) << 31))
     return set_error(MOTIF_ERR_UNSUPPORTED, "gdn_chunk_bwd: too many chunks");
   const size_t need = motif_gdn_chunk_bwd_workspace_bytes(B, H, L, dk, dv);
   if (!workspace || workspace_bytes < need)

@@ -127,3 +127,18 @@ def test_operator_scan_depths(N, dk, dv, shift, transpose):
         M = A[:, :, n].double().cpu()
         ref = (M.transpose(-1, -2) if transpose else M) @ ref + Q[:, :, n].double().cpu()
     assert (S.double().cpu() - ref).abs().max() <= 2 ** -23 * (dk / 4 + 8) * ref.abs().max()
+
+
+def test_more_batch_rows_than_a_grid_dimension():
+    '''65540 one-step rows: the rows on both sides of the launch limit as in a call of their own.'''
+    g = torch.Generator(device=DEV).manual_seed(3)
+    r = lambda *s: torch.randn(65540, 1, 1, *s, generator=g, device=DEV)  # noqa: E731
+    x = [r(64), r(64), r(64), torch.sigmoid(r()), -torch.rand(65540, 1, 1, generator=g, device=DEV)]
+    do = r(64)
+
+    def grads(rows):
+        ts = [t[rows].requires_grad_() for t in x]
+        return torch.autograd.grad(chunk_gated_delta_rule(*ts)[0], ts, do[rows])
+    whole = grads(slice(None))
+    for rows in (slice(0, 3), slice(65533, 65540)):
+        assert all(torch.equal(a[rows], b) for a, b in zip(whole, grads(rows)))
