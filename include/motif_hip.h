@@ -146,7 +146,8 @@ int motif_gdn_opscan_pair_f32(const float *A, const float *Hn, const float *S0, 
  * _PrepareChunksFunction.backward, _FusedScanFunction.backward and the output combination's
  * gradient (motif/ops/gated_deltanet.py:180-260, :727-765, :830-855).  dk == 64, dv in
  * {64, 128}; dtype fp32 or bf16 for every tensor; unit feature strides, rows of q, k, v and
- * dout on four-element boundaries; 16-byte aligned workspace.
+ * dout on four-element boundaries, row strides of those and of dq, dk, dv from the row's length
+ * up to (not including) 2^23 elements; at most 65535 heads; 16-byte aligned workspace.
  */
 size_t motif_gdn_chunk_bwd_workspace_bytes(int B, int H, int L, int dk, int dv);
 int motif_gdn_chunk_bwd(const void *q, int64_t q_sb, int64_t q_sh, int64_t q_st,
